@@ -28,6 +28,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
@@ -725,8 +726,26 @@ __device__ __forceinline__ void store_tile(float* dst, int ld, const Tile& src, 
     }
 }
 
+// 16-byte accesses at agent scope (sc1) of a wave-uniform base and a per-lane byte offset. A load reads past this CU's
+// L1 (which holds lines other workgroups have since rewritten; nothing invalidates it in the XCD-local hand-offs); a
+// store is written through the XCD's L2, so that a reader on another XCD needs no write-back of that L2.
+constexpr int AUX_SC1 = 16;
+__device__ __forceinline__ float4 load16_agent(const float* base, uint32_t off, uint32_t bytes) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        uniform_ptr(base), (short)0, (int)__builtin_amdgcn_readfirstlane(bytes), BUF_RSRC_WORD3);
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, AUX_SC1);
+    return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3]));
+}
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store16_agent(float* base, uint32_t off, uint32_t bytes, const float4 v) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        uniform_ptr(base), (short)0, (int)__builtin_amdgcn_readfirstlane(bytes), BUF_RSRC_WORD3);
+    const u32x4 q = {__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)};
+    __builtin_amdgcn_raw_buffer_store_b128(q, rs, (int)off, 0, AUX_SC1);
+}
+
 // the half of store_tile_op's packed layout that holds rows 16 h .. 16 h + 15, by one wavefront
-__device__ __forceinline__ void store_tile_op_half(float* dst, const Tile& src, int h, int lane) {
+__device__ __forceinline__ void store_tile_op_half(float* dst, const Tile& src, int h, int lane, bool wt) {
     for (int u = 0; u < 2; ++u) {
         const int e = 4 * (32 * u + (lane >> 1)) + 2 * h + (lane & 1);   // e & 3 = 2 h + (0 or 1): cb = h
         const int ln = e >> 2, kk0 = 4 * (e & 1), l16 = ln & 15, lk = ln >> 4;
@@ -735,7 +754,8 @@ __device__ __forceinline__ void store_tile_op_half(float* dst, const Tile& src, 
         v.y = src[16 * h + l16][4 * (kk0 + 1) + lk];
         v.z = src[16 * h + l16][4 * (kk0 + 2) + lk];
         v.w = src[16 * h + l16][4 * (kk0 + 3) + lk];
-        *reinterpret_cast<float4*>(dst + 4 * e) = v;
+        if (wt) store16_agent(dst, 16u * (uint32_t)e, 4u * CB * CB, v);
+        else *reinterpret_cast<float4*>(dst + 4 * e) = v;
     }
 }
 
@@ -753,15 +773,17 @@ __device__ __forceinline__ void store_tile_half(float* dst, int ld, const Tile& 
 // lane, contiguous: dst[16 lane + 8 cb + kk] = T[16 cb + (lane & 15)][4 kk + (lane >> 4)], at pair index
 // a (a + 1) / 2 + b of the packed factor (1024 floats per block).
 __device__ __forceinline__ int op_pair(int a, int b) { return a * (a + 1) / 2 + b; }
-__device__ __forceinline__ void store_tile_op(float* dst, const Tile& src, int t = -1, int nthr = 256) {
-    for (int e = (t < 0 ? (int)threadIdx.x : t); e < 256; e += nthr) {
+// wt: written through the L2 (a factorisation on one XCD, whose solve runs on all of them)
+__device__ __forceinline__ void store_tile_op(float* dst, const Tile& src, int t, int nthr, bool wt) {
+    for (int e = t; e < 256; e += nthr) {
         const int lane = e >> 2, h = e & 3, cb = h >> 1, kk0 = 4 * (h & 1), l16 = lane & 15, lk = lane >> 4;
         float4 v;
         v.x = src[16 * cb + l16][4 * (kk0 + 0) + lk];
         v.y = src[16 * cb + l16][4 * (kk0 + 1) + lk];
         v.z = src[16 * cb + l16][4 * (kk0 + 2) + lk];
         v.w = src[16 * cb + l16][4 * (kk0 + 3) + lk];
-        *reinterpret_cast<float4*>(dst + 4 * e) = v;
+        if (wt) store16_agent(dst, 16u * (uint32_t)e, 4u * CB * CB, v);
+        else *reinterpret_cast<float4*>(dst + 4 * e) = v;
     }
 }
 
@@ -796,7 +818,8 @@ __device__ __forceinline__ void load_tiles(Tile* dst, int n, int ld, uint32_t di
             }
 }
 
-// As load_tiles without shifts, tile q from srcf(q) with row stride ldf(q) into dstf(q)
+// As load_tiles without shifts, tile q from srcf(q) with row stride ldf(q) into dstf(q), with agent-scope loads (tiles
+// that other workgroups of the launch stored)
 template <int NMAX, int NTHR, class DstF, class SrcF, class LdF>
 __device__ __forceinline__ void load_tiles_to(int n, int t, DstF dstf, SrcF srcf, LdF ldf) {
     constexpr int PER = 256 / NTHR;
@@ -807,7 +830,8 @@ __device__ __forceinline__ void load_tiles_to(int n, int t, DstF dstf, SrcF srcf
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
                 const int e = t + u * NTHR, row = e >> 3, c4 = e & 7;
-                v[q][u] = *reinterpret_cast<const float4*>(srcf(q) + (size_t)row * ldf(q) + 4 * c4);
+                const uint32_t ld = (uint32_t)ldf(q);
+                v[q][u] = load16_agent(srcf(q), 4u * ((uint32_t)row * ld + 4u * (uint32_t)c4), 4u * (31u * ld + CB));
             }
 #pragma unroll
     for (int q = 0; q < NMAX; ++q)
@@ -985,9 +1009,10 @@ __device__ __forceinline__ void update32_wave(Tile& C, const Tile& Pi, const Til
     update32_wave_q<LOWER ? 0xD : 0xF>(C, C, Pi, Pk);
 }
 
-// Poll an agent-scope flag until it holds `ep` (bounded), then acquire. Called by one lane.
+// Poll an agent-scope flag until it holds `ep` (bounded), then acquire (local: no cache invalidation; the data the
+// flag covers is read with agent-scope loads). Called by one lane.
 __device__ __forceinline__ void wait_flag(const uint32_t* f, uint32_t ep, uint32_t* err, bool& dead,
-                                          uint32_t lim = SPIN_LIMIT) {
+                                          uint32_t lim = SPIN_LIMIT, bool local = false) {
     uint32_t n = 0;
     while (!dead && __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != ep) {
         if (++n > lim) {
@@ -997,14 +1022,15 @@ __device__ __forceinline__ void wait_flag(const uint32_t* f, uint32_t ep, uint32
         }
         __builtin_amdgcn_s_sleep(1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (local) asm volatile("" ::: "memory");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
 // Poll up to 64 agent-scope flags at once, each lane watching its own (`mine`; nullptr: nothing to wait for), until
 // all hold `ep` (bounded), then acquire. Called by a whole wavefront; costs one round trip after the last publication
 // instead of one per flag.
 __device__ __forceinline__ void wait_flags_wave(const uint32_t* mine, uint32_t ep, uint32_t* err, bool& dead,
-                                                uint32_t lim) {
+                                                uint32_t lim, bool local) {
     const int lane = threadIdx.x & 63;
     uint32_t polls = 0;
     while (!dead) {
@@ -1017,7 +1043,8 @@ __device__ __forceinline__ void wait_flags_wave(const uint32_t* mine, uint32_t e
         }
         __builtin_amdgcn_s_sleep(1);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (local) asm volatile("" ::: "memory");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
 // Publish: the calling lane's wave (or, after a workgroup sync, the workgroup) has its stores issued. release()
@@ -1036,6 +1063,25 @@ __device__ __forceinline__ void set_flag(uint32_t* f, uint32_t ep) {
 __device__ __forceinline__ void publish_flag(uint32_t* f, uint32_t ep) {
     release();
     set_flag(f, ep);
+}
+// The same between workgroups that share an XCD's L2 (local): the stores are complete -- in that L2 -- once vmcnt says
+// so, and the flag is stored there too (the agent-scope polls read past the CUs' L1 and find it in the L2). Other
+// XCDs see neither until the kernel ends, so a flag that workgroups elsewhere may be polling is set with set_flag.
+__device__ __forceinline__ void release_to(bool local) {
+    if (local) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+    } else {
+        release();
+    }
+}
+__device__ __forceinline__ void set_flag_to(uint32_t* f, uint32_t v, bool local) {
+    if (local) __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else set_flag(f, v);
+}
+// the XCD this workgroup runs on
+__device__ __forceinline__ uint32_t xcc_id() {
+    return __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));   // HW_REG_XCC_ID, 4 bits
 }
 
 // Barrier of some waves of a workgroup while the others keep running: an LDS counter that each participating
@@ -1314,8 +1360,18 @@ size_t chol_lds_bytes(int r, int w) {
 // column k at the release that opens step k+2 (its stores of column k's operands completed during step k+1), column
 // nb-2 at a release of its own in the last step, and column nb-1 (Li_{nb-1} alone) right after the last tile factor.
 // Column k is complete at 1 + max(0, nb - 4 - k) credits; the counters start at zero.
-static_assert(chol_workgroups(CH_MAXROW, OWNER_W) <= FLAG_STRIDE - CH_MAXROW * (CH_MAXROW + 1),
-              "a call counter per Cholesky workgroup after the panel and hand-over flags");
+//
+// One XCD (local). The hand-offs are chains of short messages between CUs, and what a message costs depends on where
+// the two CUs are: measured as a round trip of two workgroups with 8 KB each way, 2.8 us (3.7 with other workgroups
+// writing) across XCDs, where the producer must write its L2 back and the consumer invalidate its own, and 1.26 us
+// within one XCD, where the L2 is the common memory: the stores' completion, a flag in the L2, and loads that pass by
+// the L1. So the launch places the workgroups of a factorisation on one XCD when they fit there (launch index
+// congruent mod 8), and they check where they are: each owner part posts its XCD at its start, workgroup 0 compares
+// them during step 0 and says which protocol the call takes in bit 0 of every flag (the first flag an owner waits
+// for, (0, 0), is stored for all XCDs to see). What the solve reads from other XCDs, the packed operands, is then
+// written through the L2 when it is stored, so no L2 write-back is left in the kernel.
+static_assert(2 * chol_workgroups(CH_MAXROW, OWNER_W) <= FLAG_STRIDE - CH_MAXROW * (CH_MAXROW + 1),
+              "a call counter and an arrival word per Cholesky workgroup after the panel and hand-over flags");
 
 __device__ __forceinline__ void credit(uint32_t* colcnt, int k) {
     if (colcnt != nullptr) __hip_atomic_fetch_add(colcnt + (size_t)k * CC_STRIDE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1326,7 +1382,7 @@ template <bool STAMP>
 __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A, int r, const double* __restrict__ npart,
                                           int nnp, float alpha, float tau_rel, float* L, float* Li, float* Lp,
                                           uint32_t* bar, uint32_t* flags, float* scal, uint64_t* stamps, uint32_t lim,
-                                          uint32_t* colcnt, int ow, const float* tau_ptr = nullptr) {
+                                          uint32_t* colcnt, int ow, int ngrid, const float* tau_ptr = nullptr) {
     extern __shared__ float4 chol_lds[];
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int nb = r / CB;
@@ -1345,10 +1401,11 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
     uint32_t* flagL = flags;
     uint32_t* flagT = flags + nb * nb;
     uint32_t* cnt = flags + nb * nb + nb;
+    uint32_t* arr = cnt + ngrid;           // arrival words: (call number, XCD) of each owner part
     bool dead = false;
     if (STAMP && b == 0 && tid == 0) stamps[0] = stamp_clock();
-    const uint32_t ep = cnt[b] + 1;        // this call's number (every workgroup runs every call)
-    // misc: [0..2] nrm, shift, tau; workgroup 0's LDS words: [4] the row wavefronts' barrier counter, [5] the last step
+    const uint32_t calls = cnt[b];         // (read first, used only once the first tiles are here)
+    // misc: [0..2] nrm, shift, tau, [3] local; workgroup 0's LDS words: [4] the row wavefronts' barrier counter, [5] the last step
     // whose L(j+2, j) is formed, [6] the halves of L(j+2, j-1) formed, [7] the tile factor's pairs done; [32..63] the tile factor's diagonal (piv q),
     // [64..127] its per-pair scalars
     float* misc = reinterpret_cast<float*>(chol_lds);
@@ -1382,6 +1439,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
         }
         for (int off = 32; off >= 1; off >>= 1) s = s + __shfl_down(s, off);
         if (lane == 0) {
+            reinterpret_cast<uint32_t*>(misc)[3] = 0u;
             reinterpret_cast<uint32_t*>(misc)[4] = 0u;
             reinterpret_cast<uint32_t*>(misc)[5] = 0u;
             reinterpret_cast<uint32_t*>(misc)[6] = 0u;
@@ -1409,6 +1467,9 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
         }
     }
     __syncthreads();
+    const uint32_t ep = calls + 1;         // this call's number (every workgroup runs every call)
+    bool local = false;                    // this call's protocol (see above), known after workgroup 0's first flag
+    uint32_t fv = 0;                       // then the call's flag value: 2 ep + local
     float* pq = misc + 32;
 
     if (b == 0) {
@@ -1434,19 +1495,41 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
             const int q = j & 1;
             const size_t o = (size_t)CB * j;
             if (lane == 0) {
-                publish_flag(flagL + j * nb + j, ep);
+                release_to(local);
+                if (j == 0) set_flag(flagL, fv);   // (for every XCD: the owners do not know the protocol yet)
+                else set_flag_to(flagL + j * nb + j, fv, local);
                 // the release covers column j-1's operands (stored in step j); column nb-2 is credited in the last
                 // step, column nb-1 by wave 0
                 if (j >= 1 && j < nb - 1) credit(colcnt, j - 1);
             }
             store_tile_lower(L + o * r + o, r, z.dl[q], false, lane, 64);
-            store_tile_op(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[q], lane, 64);
-            if (j + 1 < nb) store_tile_op(Lp + (size_t)op_pair(j + 1, j) * CB * CB, z.P1[q], lane, 64);
+            store_tile_op(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[q], lane, 64, local);
+            if (j + 1 < nb) store_tile_op(Lp + (size_t)op_pair(j + 1, j) * CB * CB, z.P1[q], lane, 64, local);
             if (j + 2 < nb) {
                 wait_lds(p2done, (uint32_t)j + 1, err, dead, lim);   // L(j+2, j), formed by the look-ahead
                 store_tile(L + (o + 2 * CB) * r + o, r, z.P2[q], lane, 64);
-                store_tile_op(Lp + (size_t)op_pair(j + 2, j) * CB * CB, z.P2[q], lane, 64);
+                store_tile_op(Lp + (size_t)op_pair(j + 2, j) * CB * CB, z.P2[q], lane, 64, local);
             }
+        };
+        // wave 3, step 0: the XCD of every owner part, once all have posted theirs
+        auto find_protocol = [&]() {
+            bool same = true;
+            for (int b0 = 1; b0 < ngrid; b0 += 64) {
+                const int q = b0 + lane;
+                uint32_t v = 0, polls = 0;
+                while (!dead) {
+                    v = q < ngrid ? __hip_atomic_load(arr + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+                    const bool ok = q >= ngrid || (v >> 4) == (ep & 0x0fffffffu);
+                    if (__all(ok)) break;
+                    if (++polls > lim) {
+                        if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        dead = true;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+                same = same && __all(q >= ngrid || (v & 15u) == xcc_id());
+            }
+            if (lane == 0) reinterpret_cast<uint32_t*>(misc)[3] = (same && !dead) ? 1u : 0u;
         };
         // Waves 0 and 7 take turns: at step j one factors T(j, j) (wave 0 at even j), the other forms tile row j+1's
         // look-ahead beside it and so ends the step holding T(j+1, j+1) through block j -- the next step's tile, in
@@ -1465,8 +1548,8 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 if (STAMP && lane == 0) stamps[4 + 4 * j] = stamp_clock();
                 if (colcnt != nullptr && j == nb - 1) {
                     // the last column of the factor is Li_{nb-1} alone: packed, released and credited at once
-                    store_tile_op(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[p], lane, 64);
-                    release();
+                    store_tile_op(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[p], lane, 64, local);
+                    release_to(local);
                     if (lane == 0) credit(colcnt, j);
                 }
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this step's Li_j stored
@@ -1489,9 +1572,10 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this step's L(j+1, j) stored
             } else if (w == 3) {
                 // wave 3 publishes the previous step
-                if (j >= 1) publish(j - 1);
+                if (j == 0) find_protocol();
+                else publish(j - 1);
                 if (colcnt != nullptr && j == nb - 1 && nb >= 2) {   // column nb-2's operands, stored just now
-                    release();
+                    release_to(local);
                     if (lane == 0) credit(colcnt, nb - 2);
                 }
                 if (STAMP && lane == 0) stamps[2 + 5 * nb + j] = stamp_clock();
@@ -1511,7 +1595,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                     load_tiles<4, 256>(&R2[t0], 4 - t0, r, 1u << (3 - t0), shift, wl,
                                        [&](int q) { return rowp + CB * (j - 1 + t0 + q); });
                 } else {
-                    if (lane == 0) wait_flag(flagT + i2, ep, err, dead, lim);
+                    if (lane == 0) wait_flag(flagT + i2, fv, err, dead, lim, local);
                     if (STAMP && w == 1 && lane == 0) stamps[2 + 6 * nb + j] = stamp_clock();
                     __builtin_amdgcn_wave_barrier();
                     // each wavefront fetches the parts of row j+2 that it alone reads and updates below: waves 1 and
@@ -1524,15 +1608,17 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                     const float* s3 = rowp + CB * (j + 2);
                     const bool quad = !side2 || hf == 0;
                     const int qa = side2 ? 1 : hf, qb = side2 ? 0 : hf;
+                    const uint32_t tb = 4u * (31u * (uint32_t)r + CB);   // bytes of a tile's rows
                     float4 v[5];
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const int e = lane + 64 * u, row = 16 * hf + (e >> 3), c4 = e & 7;
-                        v[u] = *reinterpret_cast<const float4*>(s0 + (size_t)row * r + 4 * c4);
-                        v[2 + u] = *reinterpret_cast<const float4*>(s1 + (size_t)row * r + 4 * c4);
+                        const uint32_t off = 4u * ((uint32_t)row * (uint32_t)r + 4u * (uint32_t)c4);
+                        v[u] = load16_agent(s0, off, tb);
+                        v[2 + u] = load16_agent(s1, off, tb);
                     }
                     const int qrow = 16 * qa + (lane >> 2), qc4 = 4 * qb + (lane & 3);
-                    if (quad) v[4] = *reinterpret_cast<const float4*>(s3 + (size_t)qrow * r + 4 * qc4);
+                    if (quad) v[4] = load16_agent(s3, 4u * ((uint32_t)qrow * (uint32_t)r + 4u * (uint32_t)qc4), tb);
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const int e = lane + 64 * u, row = 16 * hf + (e >> 3), c4 = e & 7;
@@ -1559,7 +1645,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                         // its half for the output and the later kernels (the owners form their own copy)
                         const size_t o = (size_t)CB * (j - 1);
                         store_tile_half(L + (o + 3 * CB) * r + o, r, z.C2[p], hf, lane);
-                        store_tile_op_half(Lp + (size_t)op_pair(j + 2, j - 1) * CB * CB, z.C2[p], hf, lane);
+                        store_tile_op_half(Lp + (size_t)op_pair(j + 2, j - 1) * CB * CB, z.C2[p], hf, lane, local);
                     } else if (j >= 2) {                                               // T(j+2, j+1), block j-2
                         if (hf) update32_wave_q<0xC>(R2[2], R2[2], R2[4], z.C2[pp]);
                         else update32_wave_q<0x3>(R2[2], R2[2], R2[4], z.C2[pp]);
@@ -1590,17 +1676,24 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                         }
                     }
                 }
+                // T(j+2, j) and the packed L(j+2, j-1) are stored (in agent mode wave 3's release covers them)
+                if (!side2) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
                 if (STAMP && w == 1 && lane == 0) stamps[2 + 4 * nb + j] = stamp_clock();
             }
             __syncthreads();
+            if (j == 0) {
+                local = reinterpret_cast<uint32_t*>(misc)[3] != 0u;
+                fv = 2 * ep + (local ? 1u : 0u);
+            }
             // start the L2 write-back of this step's stores now; the publication at the next step's start then
             // finds the lines clean
-            if (w == 4) asm volatile("buffer_wbl2 sc1" ::: "memory");
+            if (w == 4 && !local) asm volatile("buffer_wbl2 sc1" ::: "memory");
             if (STAMP && tid == 0) stamps[2 + 4 * j] = stamp_clock();
         }
         if (w == 3) publish(nb - 1);
         if (STAMP && tid == 0) stamps[1 + 4 * nb] = stamp_clock();
     } else {
+        if (tid == 0) set_flag(arr + b, (ep << 4) | xcc_id());
         // Owner part: tile row i, tiles T(i, s..e-1) in LDS. rt[k - s] = T(i, k); pn[k - s] = L(k, j) of the current
         // column block for the part's columns k < i; li = Li_j; pin = L(i, j) when another part of the row holds
         // T(i, j). Each part runs blocks j until its tiles are done: the last part (which holds T(i, i)) to block
@@ -1643,9 +1736,29 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 } else if (lane == nk + 1 && !mine && j >= 1) {
                     f = flagL + i * nb + j;
                 }
-                wait_flags_wave(f, ep, err, dead, lim);
+                if (j == 0) {
+                    // the call's first flag, (0, 0) alone, in either protocol's value
+                    uint32_t polls = 0, got = 0;
+                    while (!dead) {
+                        got = __hip_atomic_load(flagL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if ((got >> 1) == (ep & 0x7fffffffu)) break;
+                        if (++polls > lim) {
+                            if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            dead = true;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    if (lane == 0) reinterpret_cast<uint32_t*>(misc)[3] = dead ? 0u : got & 1u;
+                    if (dead || (got & 1u) == 0u) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                } else {
+                    wait_flags_wave(f, fv, err, dead, lim, local);
+                }
             }
             __syncthreads();
+            if (j == 0) {
+                local = reinterpret_cast<uint32_t*>(misc)[3] != 0u;
+                fv = 2 * ep + (local ? 1u : 0u);
+            }
             if (hst) stamps[2 + 10 * nb + 6 * i] = stamp_clock();
             if (bst) bs[0] = stamp_clock();
             // one batch: Li_j; per column k, the finished L(j+1, j) or T(k, j) through block j-1; T(i, j) into pin
@@ -1672,7 +1785,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
             if (mine) {
                 // L(i, j): the output, and its packed form for the solve (released below, with the column credit)
                 if (q4) store_tile(L + (size_t)CB * i * r + (size_t)CB * j, r, lij);
-                else store_tile_op(Lp + (size_t)op_pair(i, j) * CB * CB, lij, tid - 256, 256);
+                else store_tile_op(Lp + (size_t)op_pair(i, j) * CB * CB, lij, tid - 256, 256, local);
             } else if (hand && q4) {
                 // workgroup 0 reads L(i, i-4) with the handed-over row: this part's own copy (the same bits as the
                 // holder's), stored before the hand-over
@@ -1747,7 +1860,8 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 __syncthreads();
                 if (hst) stamps[7 + 10 * nb + 6 * i] = stamp_clock();
                 if (tid == 0) {
-                    publish_flag(flagT + i, ep);
+                    release_to(local);
+                    set_flag_to(flagT + i, fv, local);
                     if (mine) credit(colcnt, j);   // L(i, i-4)'s packed form
                 }
                 if (hst) stamps[5 + 10 * nb + 6 * i] = stamp_clock();
@@ -1757,9 +1871,9 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 const bool pub = j + 1 >= s && j + 1 < e && j + 1 <= i - 4;
                 if (pub) store_tile(A + (size_t)CB * i * r + (size_t)CB * (j + 1), r, rt[j + 1 - s], lane, 64);
                 if (pub || mine) {
-                    release();
+                    release_to(local);
                     if (lane == 0) {
-                        if (pub) set_flag(flagL + i * nb + j + 1, ep);
+                        if (pub) set_flag_to(flagL + i * nb + j + 1, fv, local);
                         if (mine) credit(colcnt, j);
                     }
                 }
@@ -1771,15 +1885,49 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
     if (tid == 0) cnt[b] = ep;
 }
 
+// The Cholesky workgroup b of matrix z at launch index idx, or -1. Matrices m q .. m q + m - 1 have their `grid`
+// workgroups at the indices m (q grid + b) + k: with m = NXCD the hardware's round robin puts a matrix on one XCD, with
+// m = 1 its workgroups are spread over the XCDs. An index that is no Cholesky workgroup (a gap of a last group of
+// fewer than m matrices, or past them all) gets its rank among such indices in `other`.
+constexpr int NXCD = 8;
+static_assert(NXCD == 8, "chol_role's shift");
+// (Divisions only where a launch has more than one group of matrices: at the head of every workgroup they cost ~1 us.)
+__device__ __forceinline__ int chol_role(int idx, int grid, int nz, int m, int& z, int& other) {
+    const int sh = m == NXCD ? 3 : 0, s = idx >> sh, k = idx & (m - 1);
+    int q = 0;
+    if (nz > m) {
+        q = s / grid;
+        if (m * q >= nz) {
+            other = idx - nz * grid;
+            return -1;
+        }
+    } else if (s >= grid) {
+        other = idx - nz * grid;
+        return -1;
+    }
+    z = m * q + k;
+    if (z < nz) return s - q * grid;
+    const int nlast = nz - m * q;
+    other = (s - q * grid) * (m - nlast) + k - nlast;
+    return -1;
+}
+// launch indices of the Cholesky's workgroups with `others` further ones
+int chol_launch_size(int grid, int nz, int m, int others) {
+    return std::max((nz + m - 1) / m * m * grid, nz * grid + others);
+}
+
 // tau_ptr (nnp == 0 only; may be null): the absolute pivot floor read from device memory instead of tau_rel (chol32
 // with tau as a device tensor, kchol.py:24-28: no host synchronisation)
 template <bool STAMP>
 __global__ __launch_bounds__(512) void k_chol(float* A, int r, const double* __restrict__ npart, int nnp, float alpha,
                                               float tau_rel, float* L, float* Li, float* Lp, uint32_t* bar,
                                               uint32_t* flags, float* scal, uint64_t* stamps, uint32_t lim, int ow,
-                                              const float* tau_ptr) {
-    chol_body<STAMP>(blockIdx.x, blockIdx.z, A, r, npart, nnp, alpha, tau_rel, L, Li, Lp, bar, flags, scal, stamps,
-                     lim, nullptr, ow, tau_ptr);
+                                              int grid, int nz, int m, const float* tau_ptr) {
+    int z = 0, other = 0;
+    const int b = chol_role(blockIdx.x, grid, nz, m, z, other);
+    if (b < 0) return;
+    chol_body<STAMP>(b, z, A, r, npart, nnp, alpha, tau_rel, L, Li, Lp, bar, flags, scal, stamps, lim, nullptr, ow, grid,
+                     tau_ptr);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -2174,7 +2322,7 @@ __device__ __forceinline__ void trsm_wave_body(const int g, const int z, const M
 // are dispatched first and never wait on a solve workgroup). Pointers address matrix 0 of the launch.
 struct CholArgs {
     float* A; const double* npart; float* L; float* Li; float* Lp; uint32_t* bar; uint32_t* flags; float* scal;
-    uint32_t* colcnt; float alpha, tau_rel; int r, nnp, nz, grid, ow; uint32_t lim;   // ow: owner part width
+    uint32_t* colcnt; float alpha, tau_rel; int r, nnp, nz, grid, m, ow; uint32_t lim;   // m: chol_role; ow: owner part width
 };
 struct SolveArgs {
     MatsIn A; MatsOut Y; const uint32_t* amax_part; const float* Z; float* scal; long lda, ldz, ldy; float eps;
@@ -2185,18 +2333,20 @@ struct SolveArgs {
 // with NBC = RB column blocks (eight row blocks per workgroup).
 template <bool PASS1, int Q, int RB>
 __global__ __launch_bounds__(64 * TRSM_NW) void k_chol_solve(const CholArgs c, const SolveArgs t) {
-    const int nchol = c.nz * c.grid;
-    if ((int)blockIdx.x < nchol) {
-        chol_body<false>(blockIdx.x % c.grid, blockIdx.x / c.grid, c.A, c.r, c.npart, c.nnp, c.alpha, c.tau_rel, c.L,
-                         c.Li, c.Lp, c.bar, c.flags, c.scal, nullptr, c.lim, c.colcnt, c.ow);
+    int z = 0, b = 0;
+    const int cb = chol_role(blockIdx.x, c.grid, c.nz, c.m, z, b);
+    if (cb >= 0) {
+        chol_body<false>(cb, z, c.A, c.r, c.npart, c.nnp, c.alpha, c.tau_rel, c.L, c.Li, c.Lp, c.bar, c.flags, c.scal,
+                         nullptr, c.lim, c.colcnt, c.ow, c.grid);
         return;
     }
-    const int b = blockIdx.x - nchol;
+    if (b >= c.nz * t.nrb) return;   // a gap that holds no solve workgroup
+    const int zs = c.nz == 1 ? 0 : b / t.nrb, rb = b - zs * t.nrb;
     if constexpr (Q == 0)
-        trsm_wave_body<PASS1, RB>(b % t.nrb, b / t.nrb, t.A, t.lda, t.K, t.wpg, t.amax_part, t.Z, t.ldz, t.eps, c.Lp, t.Y,
+        trsm_wave_body<PASS1, RB>(rb, zs, t.A, t.lda, t.K, t.wpg, t.amax_part, t.Z, t.ldz, t.eps, c.Lp, t.Y,
                                   t.ldy, t.scal, c.colcnt, c.bar, c.lim);
     else
-        trsm_body<PASS1, Q, RB, true>(b % t.nrb, b / t.nrb, t.A, t.lda, t.K, c.r, t.amax_part, t.Z, t.ldz, t.eps,
+        trsm_body<PASS1, Q, RB, true>(rb, zs, t.A, t.lda, t.K, c.r, t.amax_part, t.Z, t.ldz, t.eps,
                                       c.Lp, t.Y, t.ldy, t.scal, c.colcnt, c.bar, c.lim);
 }
 
@@ -2730,6 +2880,7 @@ struct spanqr_plan {
     bool gram_short = false;  // one-launch Gram over upper 32x32 tiles (k_gram32) instead of split Gram + reduction
     int nnp = 0;              // norm partials per matrix the Gram writes (16 per 64x64 tile, or 1 per 32x32 tile)
     int owner_w = OWNER_W;    // tiles per Cholesky owner part at most
+    int chol_m = 1;           // NXCD: each matrix's Cholesky workgroups on one XCD; 1: spread (chol_role)
     bool trsm_rows = false;   // solve with a wavefront pair per 16 rows (k_trsm_rows) instead of k_trsm
     int solve_rb = 0;         // row blocks per solve workgroup in the Cholesky's launch (0: separate launches)
     int solve_nrb = 0;        // solve workgroups per matrix there
@@ -2908,13 +3059,13 @@ int launch_chol(spanqr_plan* p, float alpha, float tau, float* scal, hipStream_t
         uint32_t* bar = p->bar + (size_t)z0 * BAR_STRIDE;
         uint32_t* flags = p->flags + (size_t)z0 * FLAG_STRIDE;
         float* sc = scal ? scal + (size_t)z0 * SCAL_STRIDE : nullptr;
-        const dim3 grid(p->chol_grid, 1, nz);
+        const dim3 grid(chol_launch_size(p->chol_grid, nz, p->chol_m, 0));
         if (stamp)
             k_chol<true><<<grid, 512, lds, st>>>(A, p->r, np, nnp, alpha, tau, L, Li, Lp, bar, flags, sc, p->stamps,
-                                                 g_spin_limit, p->owner_w, tau_ptr);
+                                                 g_spin_limit, p->owner_w, p->chol_grid, nz, p->chol_m, tau_ptr);
         else
             k_chol<false><<<grid, 512, lds, st>>>(A, p->r, np, nnp, alpha, tau, L, Li, Lp, bar, flags, sc, p->stamps,
-                                                  g_spin_limit, p->owner_w, tau_ptr);
+                                                  g_spin_limit, p->owner_w, p->chol_grid, nz, p->chol_m, tau_ptr);
         HIPCHK(hipGetLastError());
     }
     return SPANQR_OK;
@@ -3100,6 +3251,7 @@ int launch_chol_solve(spanqr_plan* p, float alpha, float tau, float* scal, hipSt
         c.nnp = nnp;
         c.nz = nz;
         c.grid = p->chol_grid;
+        c.m = p->chol_m;
         c.ow = p->owner_w;
         c.lim = g_spin_limit;
         SolveArgs t{};
@@ -3117,7 +3269,7 @@ int launch_chol_solve(spanqr_plan* p, float alpha, float tau, float* scal, hipSt
         t.K = p->K;
         t.nrb = p->solve_nrb;
         t.wpg = p->solve_wpg;
-        const dim3 grid(nz * (p->chol_grid + p->solve_nrb));
+        const dim3 grid(chol_launch_size(p->chol_grid, nz, p->chol_m, nz * p->solve_nrb));
         if (pass1) launch_fused<true>(q, q ? p->solve_rb : p->r / CB, grid, lds, st, c, t);
         else launch_fused<false>(q, q ? p->solve_rb : p->r / CB, grid, lds, st, c, t);
         HIPCHK(hipGetLastError());
@@ -3299,42 +3451,45 @@ int plan_device_setup(spanqr_plan* p, int device) {
         if ((size_t)maxsh < need)
             return fail(SPANQR_EHIP, "the solve needs %zu bytes of LDS per workgroup, device allows %d", need, maxsh);
     }
-    int occ = 0, cus = 0;
+    int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     p->cus = cus;
-    // The owner part width: OWNER_W for one matrix; for a batch, the narrowest of 6, 8, 12 and 16 tiles that runs
-    // the batch's Cholesky in the fewest launches (each launch needs all its workgroups resident at once, within
-    // three quarters of the device: the margin leaves room for work of other streams)
+    // The owner part width and the placement. A factorisation whose workgroups all fit on one XCD goes there (m =
+    // NXCD); otherwise its workgroups are spread (m = 1). One matrix takes the narrowest parts, in tiles, that fit on
+    // one XCD with at most 8 tiles (12-tile parts there: 671 us per call at 3001 x 736, 6-tile parts spread: 656), or
+    // else OWNER_W; a batch the narrowest parts that run its Cholesky in the fewest launches. Each launch
+    // needs all its workgroups resident at once: several matrices take at most 7/8 of an XCD or three quarters of the
+    // device (the margin leaves room for work of other streams).
     {
         const int widths[] = {OWNER_W, 8, 12, OWNER_WMAX};
-        int best_w = 0, best_n = 1 << 30, best_occ = 0;
-        for (int w : widths) {
-            if (p->batch == 1 && w != OWNER_W) break;
-            int o = 0;
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (const void*)k_chol<true>, 512, chol_lds_bytes(r, w)));
-            const int grid = chol_workgroups(r / CB, w);
-            if (o * cus < grid) continue;
-            int bmax = (o * cus * 3 / 4) / grid;
-            if (bmax < 1) bmax = 1;
-            const int launches = (p->batch + bmax - 1) / bmax;
-            if (launches < best_n) {
-                best_n = launches;
-                best_w = w;
-                best_occ = o;
+        int best_n = 1 << 30;
+        for (int pass = 0; pass < 2; ++pass)
+            for (int w : widths) {
+                int o = 0;
+                HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (const void*)k_chol<true>, 512, chol_lds_bytes(r, w)));
+                const int grid = chol_workgroups(r / CB, w), xcd = o * cus / NXCD;
+                int bmax;
+                if (pass == 0) {
+                    if (grid > xcd || (p->batch == 1 && w > 8)) continue;
+                    bmax = NXCD * std::max(1, xcd * 7 / 8 / grid);
+                } else {
+                    if (p->batch == 1 && best_n == 1) break;
+                    if (o * cus < grid || (p->batch == 1 && w != OWNER_W)) continue;
+                    bmax = std::max(1, (o * cus * 3 / 4) / grid);
+                }
+                const int launches = (p->batch + bmax - 1) / bmax;
+                if (launches < best_n) {
+                    best_n = launches;
+                    p->owner_w = w;
+                    p->chol_grid = grid;
+                    p->chol_m = pass == 0 ? NXCD : 1;
+                    p->chol_bmax = std::min(bmax, p->batch);
+                }
             }
-        }
-        if (best_w == 0)
+        if (best_n == 1 << 30)
             return fail(SPANQR_EHIP, "the Cholesky needs %d co-resident workgroups, device holds too few",
                         chol_workgroups(r / CB, OWNER_WMAX));
-        p->owner_w = best_w;
-        p->chol_grid = chol_workgroups(r / CB, best_w);
-        occ = best_occ;
     }
-    // a batch's launch takes at most three quarters of the device's resident capacity: the flag waits need every
-    // workgroup of a launch resident at once, and the margin leaves room for work of other streams
-    p->chol_bmax = (occ * cus * 3 / 4) / p->chol_grid;
-    if (p->chol_bmax < 1) p->chol_bmax = 1;
-    if (p->chol_bmax > p->batch) p->chol_bmax = p->batch;
     // The solve in the Cholesky's launch: enough rows per workgroup that one matrix's solve workgroups are resident
     // beside its Cholesky (one workgroup per CU: the launch's LDS is the Cholesky's); otherwise separate launches.
     // Up to one row block per CU: k_trsm's structure (eight wavefronts share a row block's column blocks); taller X at
