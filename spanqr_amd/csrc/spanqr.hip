@@ -29,6 +29,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -4272,19 +4273,34 @@ int spanqr_orth_f32_noalloc(int K, int r, const float* X, long ldx, float* Q, lo
 // ===============================================================================================================
 // fp64 clamped Cholesky (kchol.chol64, kchol.py:47-57 -> chol_f64, chol.cu:115-281 instantiated for double): the
 // tile algorithm of the fp32 factorisation in double, plus fp32 copies of L and Li (chol.cu:175-176, 215, 255).
-// Every workgroup owns one lower 32x32 tile (i, k) for the whole factorisation: it applies column blocks j < k in
-// order, each as soon as the panels L(i, j) and L(k, j) are published (fma chains over the block's 32 columns, two
-// rows x two columns per thread); then the diagonal owner factors and inverts its tile in one wavefront (the fp32
-// kernel's per-column scheme in double: the pivot from lane c's register, column broadcast through LDS), and an
-// off-diagonal owner forms its panel L(i, k) = T(i, k) Li_k^T (chain over the non-zero 16-column groups of Li_k)
-// once Li_k is published. Publication: stores, wait for them, one agent-scope release, a flag; waits are bounded
-// (an error word records a wait that gave up). Each tile waits only on tiles of earlier columns or its own column's
-// diagonal tile, so with every workgroup resident (checked when the plan is made) nothing deadlocks.
+// Workgroup 0 runs the diagonal chain and the first panel below it; every tile row i >= 2 belongs, for the whole
+// factorisation, to one or more workgroups ("parts") that hold a run of its tiles in LDS. Step j of workgroup 0: wave
+// 0 factors and inverts T(j, j) while waves 4-7 fetch T(j+1, j) and T(j+1, j+1) from row j+1's last part (through
+// block j-1) and waves 1-3 write step j-1's outputs; then L(j+1, j) = T(j+1, j) Li_j^T and T(j+1, j+1) -= L(j+1, j)
+// L(j+1, j)^T on waves 0-3 while waves 4-7 publish Li_j, then L(j+1, j). Block j of a part: the part that holds
+// T(i, j) forms and publishes L(i, j) as soon as Li_j is there; then every T(i, k), k > j, takes L(i, j) L(k, j)^T
+// (L(j+1, j) from workgroup 0, the others from row k's parts); after block i-2 the last part hands T(i, i-1..i) to
+// workgroup 0. All products are v_mfma_f64_16x16x4_f64 chains in ascending k, which round like sequential fmas.
+// What bounds it: the chain of 32-column steps, each a tile factor (a serial chain of 32 pivots) and two products on
+// one CU, and beside it the loop through row j+2's part (Li_j, panel, update, hand-over), so the workgroups of a
+// factorisation sit on one XCD where they fit and hand over through its L2 (n <= 608; the protocol of the fp32
+// factorisation, with the same check of where the workgroups are).
+// Publication: stores, wait for them, release, a flag that carries the call number; waits are bounded and the error
+// word takes the call number of a call in which one gave up. Rows wait only on earlier rows' same block and on
+// workgroup 0, which waits only on the row before the one it factors, so with every workgroup resident (checked when
+// the plan is made) nothing deadlocks.
 // ===============================================================================================================
 namespace {
 
-constexpr int C64_TS = CB + 1;
+constexpr int C64_TS = CB + 4;   // row stride in doubles: 16-byte rows, and an MFMA operand read hits every bank twice
 typedef double TileD[CB][C64_TS];
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int C64_WG0_TILES = 9;   // D[2], X, P[2], dl[2], li[2]
+constexpr int C64_MISC = 160;      // doubles in front of the tiles: the factor's column broadcasts, the protocol word
+
+__device__ __forceinline__ f64x4 mfma64(double a, double b, f64x4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
 
 __device__ __forceinline__ double readlane_d(double v, int l) {
     const uint64_t u = (uint64_t)__double_as_longlong(v);
@@ -4309,182 +4325,391 @@ __device__ __forceinline__ double rsqrt64_sw(double x) {
     return y;
 }
 
-// global 32x32 double tile (row stride ld) <-> LDS, all 256 threads, two doubles per access
-__device__ __forceinline__ void load_tile_d(TileD& dst, const double* src, long ld) {
-    for (int e = threadIdx.x; e < CB * CB / 2; e += 256) {
-        const int row = e >> 4, c2 = e & 15;
-        const double2 v = *reinterpret_cast<const double2*>(src + (size_t)row * ld + 2 * c2);
-        dst[row][2 * c2] = v.x;
-        dst[row][2 * c2 + 1] = v.y;
-    }
+// Tiles move as 512 pieces of two doubles, piece e = (row e / 16, columns 2 (e % 16), + 1); thread t of nthr takes
+// the pieces t, t + nthr, ...
+__device__ __forceinline__ double2 tile_piece(const TileD& T, int e) {
+    return *reinterpret_cast<const double2*>(&T[e >> 4][2 * (e & 15)]);
 }
-// to dst (fp64) and dstf (fp32 copy), both row stride ld; lower: zeros above the diagonal
-__device__ __forceinline__ void store_tile_d(double* dst, float* dstf, long ld, const TileD& src, bool lower) {
-    for (int e = threadIdx.x; e < CB * CB / 2; e += 256) {
-        const int row = e >> 4, c2 = e & 15;
-        double2 v;
-        v.x = (lower && 2 * c2 > row) ? 0.0 : src[row][2 * c2];
-        v.y = (lower && 2 * c2 + 1 > row) ? 0.0 : src[row][2 * c2 + 1];
-        *reinterpret_cast<double2*>(dst + (size_t)row * ld + 2 * c2) = v;
-        *reinterpret_cast<float2*>(dstf + (size_t)row * ld + 2 * c2) = make_float2((float)v.x, (float)v.y);
-    }
+__device__ __forceinline__ void put_piece(TileD& T, int e, const double2 v) {
+    *reinterpret_cast<double2*>(&T[e >> 4][2 * (e & 15)]) = v;
 }
-
-// T -= Pa Pb^T (chain over m = 0..31 from T); lower: elements above the diagonal are left (never read)
-__device__ __forceinline__ void update_d(TileD& T, const TileD& Pa, const TileD& Pb, bool lower) {
-#pragma clang fp contract(off)
-    const int r0 = 2 * (threadIdx.x >> 4), c0 = 2 * (threadIdx.x & 15);
-    double acc[2][2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int v = 0; v < 2; ++v) acc[u][v] = T[r0 + u][c0 + v];
-#pragma unroll 4
-    for (int m = 0; m < CB; ++m) {
-        const double a0 = Pa[r0][m], a1 = Pa[r0 + 1][m], b0 = Pb[c0][m], b1 = Pb[c0 + 1][m];
-        acc[0][0] = __builtin_fma(-a0, b0, acc[0][0]);
-        acc[0][1] = __builtin_fma(-a0, b1, acc[0][1]);
-        acc[1][0] = __builtin_fma(-a1, b0, acc[1][0]);
-        acc[1][1] = __builtin_fma(-a1, b1, acc[1][1]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int v = 0; v < 2; ++v)
-            if (!(lower && c0 + v > r0 + u)) T[r0 + u][c0 + v] = acc[u][v];
-    __syncthreads();
+__device__ __forceinline__ double2 load_piece(const double* src, long ld, int e) {
+    return *reinterpret_cast<const double2*>(src + (size_t)(e >> 4) * ld + 2 * (e & 15));
+}
+// the same past the L1: what another workgroup wrote in this launch
+__device__ __forceinline__ double2 load_piece_agent(const double* src, int ld, int e) {
+    const float4 v = load16_agent(reinterpret_cast<const float*>(src), (uint32_t)((e >> 4) * ld + 2 * (e & 15)) * 8u,
+                                  (uint32_t)((CB - 1) * ld + CB) * 8u);
+    return __builtin_bit_cast(double2, v);
+}
+__device__ __forceinline__ void store_piece(double* dst, long ld, int e, const double2 v) {
+    *reinterpret_cast<double2*>(dst + (size_t)(e >> 4) * ld + 2 * (e & 15)) = v;
+}
+__device__ __forceinline__ void store_piece_f(float* dst, long ld, int e, const double2 v) {
+    *reinterpret_cast<float2*>(dst + (size_t)(e >> 4) * ld + 2 * (e & 15)) = make_float2((float)v.x, (float)v.y);
+}
+// the factor's piece with zeros above the diagonal
+__device__ __forceinline__ double2 lower_piece(const TileD& T, int e) {
+    double2 v = tile_piece(T, e);
+    const int row = e >> 4, c = 2 * (e & 15);
+    if (c > row) v.x = 0.0;
+    if (c + 1 > row) v.y = 0.0;
+    return v;
 }
 
-// Out = T Li^T (chain over m < 16 (b / 16 + 1) from +0); Out may alias T
-__device__ __forceinline__ void panel_d(TileD& Out, const TileD& T, const TileD& Li) {
-#pragma clang fp contract(off)
-    const int r0 = 2 * (threadIdx.x >> 4), c0 = 2 * (threadIdx.x & 15);
-    const int mend = 16 * (c0 / 16 + 1);
-    double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-#pragma unroll 4
-    for (int m = 0; m < mend; ++m) {
-        const double a0 = T[r0][m], a1 = T[r0 + 1][m], b0 = Li[c0][m], b1 = Li[c0 + 1][m];
-        acc[0][0] = __builtin_fma(a0, b0, acc[0][0]);
-        acc[0][1] = __builtin_fma(a0, b1, acc[0][1]);
-        acc[1][0] = __builtin_fma(a1, b0, acc[1][0]);
-        acc[1][1] = __builtin_fma(a1, b1, acc[1][1]);
+// quadrant (bi, bj) of C -= Pi Pk^T (chain over m = 0..31 from C), one wavefront
+__device__ __forceinline__ void update_quad(TileD& C, const TileD& Pi, const TileD& Pk, int bi, int bj) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
+    double a[8], b[8];
+    f64x4 acc;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+        a[kk] = -Pi[16 * bi + l16][4 * kk + lk];
+        b[kk] = Pk[16 * bj + l16][4 * kk + lk];
     }
-    __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int v = 0; v < 4; ++v) acc[v] = C[16 * bi + 4 * v + lk][16 * bj + l16];
 #pragma unroll
-        for (int v = 0; v < 2; ++v) Out[r0 + u][c0 + v] = acc[u][v];
-    __syncthreads();
+    for (int kk = 0; kk < 8; ++kk) acc = mfma64(a[kk], b[kk], acc);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) C[16 * bi + 4 * v + lk][16 * bj + l16] = acc[v];
 }
 
-// Wave 0: factor the lower part of D and invert the factor (chol.cu:131-168 in double). Lanes 0..31 hold row i of D,
-// lanes 32..63 column i of the identity, which becomes column i of the inverse; column c: piv = fmax(D_cc, tau)
-// (NaN -> tau) from lane c, q = rsqrt(piv), own = R[c] q (l_i on a factor lane, x_c on an inverse lane, exactly 0
-// above its diagonal), then R[k] = fma(-own, l_k, R[k]) for k > c with l_k broadcast through LDS. The column loop
-// is a real loop (the row stays in registers, updated under k > c), which keeps the register count low. The factor's
-// diagonal entry is piv q. Writes the factor (upper triangle unspecified) to dl and the inverse to Li.
-__device__ __forceinline__ void factor_inv32_d(const TileD& D, double tau, TileD& dl, TileD& Li, double* bl, double* pq) {
+// quadrant (bi, bj) of Out = T Li^T (chain over m < 16 (bj + 1) from +0), one wavefront
+__device__ __forceinline__ void panel_quad(TileD& Out, const TileD& T, const TileD& Li, int bi, int bj) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    double a[8], b[8];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+        a[kk] = T[16 * bi + l16][4 * kk + lk];
+        b[kk] = Li[16 * bj + l16][4 * kk + lk];
+    }
+    if (bj) {
+#pragma unroll
+        for (int kk = 4; kk < 8; ++kk) {
+            a[kk] = T[16 * bi + l16][4 * kk + lk];
+            b[kk] = Li[16 + l16][4 * kk + lk];
+        }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) acc = mfma64(a[kk], b[kk], acc);
+    if (bj) {
+#pragma unroll
+        for (int kk = 4; kk < 8; ++kk) acc = mfma64(a[kk], b[kk], acc);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Out[16 * bi + 4 * v + lk][16 * bj + l16] = acc[v];
+}
+
+// One wavefront: factor the lower part of D and invert the factor (chol.cu:131-168 in double). Lanes 0..31 hold row i
+// of D, lanes 32..63 column i of the identity, which becomes column i of the inverse; column c: piv = fmax(D_cc, tau)
+// (NaN -> tau), q = rsqrt(piv), own = R[c] q (l_i on a factor lane, x_c on an inverse lane, exactly 0 above its
+// diagonal), then R[k] = fma(-own, l_k, R[k]) for k > c. The next pivot is taken first, from lane c+1's own
+// registers, so its reciprocal square root -- the serial chain -- runs beside this column's updates, whose l_k come
+// through LDS (one wavefront's LDS operations complete in order). The factor's diagonal entry is piv q. Writes the
+// factor (upper triangle unspecified) to dl and the inverse to Li; bl: 128 doubles.
+__device__ __forceinline__ void factor_inv32_d(const TileD& D, double tau, TileD& dl, TileD& Li, double* bl) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, i = lane & 31;
     const bool fl = lane < 32;
     double R[CB];
 #pragma unroll
     for (int k = 0; k < CB; ++k) R[k] = fl ? D[i][k] : (i == k ? 1.0 : 0.0);
-#pragma nounroll
+    double piv = fmax(readlane_d(R[0], 0), tau), q = rsqrt64_sw(piv), diag = 0.0;
+#pragma unroll
     for (int c = 0; c < CB; ++c) {
-        double rc = 0.0;
-#pragma unroll
-        for (int k = 0; k < CB; ++k)
-            if (k == c) rc = R[k];
-        const double piv = fmax(readlane_d(rc, c), tau);
-        const double q = rsqrt64_sw(piv);
-        const double own = (!fl && c < i) ? 0.0 : rc * q;
-        if (lane == 0) pq[c] = piv * q;
-        if (fl) bl[i] = own;
-        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int k = 0; k < CB; ++k) {
-            if (k == c) R[k] = own;
-            else if (k > c) R[k] = __builtin_fma(-own, bl[k], R[k]);
+        const double own = (!fl && c < i) ? 0.0 : R[c] * q;
+        diag = i == c ? piv * q : diag;
+        double* bc = bl + 64 * (c & 1);
+        bc[lane] = own;
+        if (c + 1 < CB) {
+            piv = fmax(readlane_d(__builtin_fma(-own, own, R[c + 1]), c + 1), tau);
+            q = rsqrt64_sw(piv);
         }
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        __builtin_amdgcn_wave_barrier();
+        R[c] = own;
+#pragma unroll
+        for (int k = c + 1; k < CB; ++k) R[k] = __builtin_fma(-own, bc[k], R[k]);
+        __builtin_amdgcn_sched_barrier(0);   // (free to mix columns, the scheduler spills)
     }
 #pragma unroll
     for (int k = 0; k < CB; ++k) {
-        if (fl) dl[i][k] = (k == i) ? pq[i] : R[k];
+        if (fl) dl[i][k] = (k == i) ? diag : R[k];
         else Li[k][i] = R[k];
     }
 }
 
-__global__ __launch_bounds__(256) void k_c64_fill(uint32_t* flags, int nf, double* L, float* Lf, int n) {
-    const size_t nn = (size_t)n * n;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < nn; e += (size_t)gridDim.x * 256) {
-        L[e] = 0.0;
-        Lf[e] = 0.0f;
-        if (e < (size_t)nf) flags[e] = 0u;
+// Tile row i >= 2 is split like the fp32 factorisation's rows; workgroup b >= 1: row i, tiles [s, e)
+__device__ inline void owner_part64(int b, int nb, int w, int& i, int& s, int& e) {
+    int q = b - 1;
+    i = 2;
+    while (i < nb - 1 && q >= row_parts(i, w)) {
+        q -= row_parts(i, w);
+        ++i;
     }
+    part_range(i, q, w, s, e);
+}
+constexpr int chol64_workgroups(int nb, int w) {
+    int n = 1;
+    for (int i = 2; i < nb; ++i) n += row_parts(i, w);
+    return n;
+}
+// a part's tiles and their panels, and a tile for Li_j or a foreign L(i, j)
+size_t chol64_lds_bytes(int n, int w) {
+    const int nb = n / CB, part = 2 * std::min(nb, w) + 1;
+    return (size_t)std::max(part, C64_WG0_TILES) * sizeof(TileD) + C64_MISC * sizeof(double);
+}
+// flag words: [nb] Li_j, [nb] L(j+1, j), [nb] hand-over of row j, [nb nb] L(i, j), then the error word and, per
+// workgroup, a call counter and an arrival word
+__host__ __device__ constexpr int chol64_err_word(int nb) { return nb * nb + 3 * nb; }
+
+// wait_flags_wave with the call number in the error word
+__device__ __forceinline__ void wait64(const uint32_t* mine, uint32_t fv, uint32_t* err, uint32_t ep, bool& dead,
+                                       uint32_t lim, bool local) {
+    uint32_t polls = 0;
+    while (!dead) {
+        const bool ok = mine == nullptr || __hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == fv;
+        if (__all(ok)) break;
+        if (++polls > lim) {
+            if ((threadIdx.x & 63) == 0) __hip_atomic_store(err, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            dead = true;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+    if (local) asm volatile("" ::: "memory");
+    else __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
-__global__ __launch_bounds__(256) void k_chol64(const double* __restrict__ G, long ldg, int n,
+__global__ __launch_bounds__(256) void k_c64_clear(uint32_t* words, int n) {
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256) words[e] = 0u;
+}
+
+constexpr int C64_OWMAX = 8;   // widest parts: 17 tiles of LDS
+
+__global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, long ldg, int n,
                                                 const double* __restrict__ taup, double* L, double* Li, float* Lf,
-                                                float* Lif, uint32_t* flags) {
-    extern __shared__ double c64_lds[];
-    TileD* tl = reinterpret_cast<TileD*>(c64_lds);
-    TileD& T = tl[0];
-    TileD& Pa = tl[1];
-    TileD& Pb = tl[2];
-    TileD& X = tl[3];
-    double* bl = c64_lds + 4 * CB * C64_TS;
-    double* pq = bl + CB;
-    const int u = blockIdx.x, nb = n / CB, nt = nb * (nb + 1) / 2;
-    int i = 0;
-    while ((i + 1) * (i + 2) / 2 <= u) ++i;
-    const int k = u - i * (i + 1) / 2;
-    uint32_t* err = flags + nt;
-    auto fidx = [](int a, int b) { return a * (a + 1) / 2 + b; };
-    bool dead = false;
-    const double tau = *taup;
-    load_tile_d(T, G + (size_t)CB * i * ldg + CB * k, ldg);
-    __syncthreads();
-    for (int j = 0; j < k; ++j) {
-        if (threadIdx.x == 0) {
-            wait_flag(flags + fidx(i, j), 1u, err, dead);
-            if (i != k) wait_flag(flags + fidx(k, j), 1u, err, dead);
+                                                float* Lif, uint32_t* flags, int grid, int m, int ow, uint32_t lim) {
+    int zz = 0, other = 0;
+    const int b = chol_role(blockIdx.x, grid, 1, m, zz, other);
+    if (b < 0) return;
+    extern __shared__ double2 c64_lds[];
+    double* misc = reinterpret_cast<double*>(c64_lds);
+    uint32_t* proto = reinterpret_cast<uint32_t*>(misc + 128);
+    TileD* tl = reinterpret_cast<TileD*>(misc + C64_MISC);
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nb = n / CB;
+    uint32_t *fD = flags, *fP = fD + nb, *fH = fP + nb, *fL = fH + nb, *err = flags + chol64_err_word(nb),
+             *cnt = err + 1, *arr = cnt + grid;
+    const uint32_t ep = cnt[b] + 1;   // this call's number (every workgroup runs every call)
+    uint32_t fv = 0;                  // the call's flag value: 2 ep + local
+    bool dead = false, local = false;
+    auto Lt = [&](int i, int k) { return L + (size_t)CB * i * n + (size_t)CB * k; };
+    auto Lft = [&](int i, int k) { return Lf + (size_t)CB * i * n + (size_t)CB * k; };
+    const double2 zero = make_double2(0.0, 0.0);
+
+    if (b == 0) {
+        TileD *D = tl, &X = tl[2], *P = tl + 3, *dl = tl + 5, *li = tl + 7;
+        const double tau = *taup;
+        put_piece(D[0], tid, load_piece(G, ldg, tid));
+        if (nb > 1) {
+            put_piece(X, tid, load_piece(G + (size_t)CB * ldg, ldg, tid));
+            put_piece(D[1], tid, load_piece(G + (size_t)CB * ldg + CB, ldg, tid));
+            store_piece(Lt(0, 1), n, tid, zero);
+            store_piece_f(Lft(0, 1), n, tid, zero);
         }
         __syncthreads();
-        load_tile_d(Pa, L + (size_t)CB * i * n + CB * j, n);
-        if (i != k) load_tile_d(Pb, L + (size_t)CB * k * n + CB * j, n);
-        __syncthreads();
-        update_d(T, Pa, i == k ? Pa : Pb, i == k);
-    }
-    if (i == k) {
-        if (threadIdx.x < 64) factor_inv32_d(T, tau, X, Pa, bl, pq);
-        __syncthreads();
-        store_tile_d(L + (size_t)CB * k * n + CB * k, Lf + (size_t)CB * k * n + CB * k, n, X, true);
-        store_tile_d(Li + (size_t)CB * k * CB, Lif + (size_t)CB * k * CB, CB, Pa, false);
+        // what only later kernels read of step j, by threads t of nthr
+        auto outputs = [&](int j, int t, int nthr) {
+            const int q = j & 1;
+            for (int e = t; e < CB * CB / 2; e += nthr) {
+                const double2 v = lower_piece(dl[q], e);
+                store_piece(Lt(j, j), n, e, v);
+                store_piece_f(Lft(j, j), n, e, v);
+                store_piece_f(Lif + (size_t)j * CB * CB, CB, e, tile_piece(li[q], e));
+                if (j + 1 < nb) store_piece_f(Lft(j + 1, j), n, e, tile_piece(P[q], e));
+            }
+        };
+        for (int j = 0; j < nb; ++j) {
+            const int q = j & 1, t4 = tid - 256;
+            if (w == 0) {
+                factor_inv32_d(D[q], tau, dl[q], li[q], misc);
+            } else if (w < 4) {
+                if (j > 0) outputs(j - 1, tid - 64, 192);
+            } else if (j > 0) {
+                if (w == 4 && lane == 0) {
+                    release_to(local);
+                    set_flag_to(fP + j - 1, fv, local);
+                }
+                if (j + 1 < nb) {
+                    wait64(lane == 0 ? fH + j + 1 : nullptr, fv, err, ep, dead, lim, local);
+                    double2 v[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        v[u] = load_piece_agent(Lt(j + 1, j + (u >> 1)), n, t4 + 256 * (u & 1));
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) put_piece(u < 2 ? X : D[1 - q], t4 + 256 * (u & 1), v[u]);
+                }
+            } else if (w == 7) {
+                // where every part is, once all have posted it
+                bool same = true;
+                for (int b0 = 1; b0 < grid; b0 += 64) {
+                    const int o = b0 + lane;
+                    uint32_t v = 0, polls = 0;
+                    while (!dead) {
+                        v = o < grid ? __hip_atomic_load(arr + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+                        if (__all(o >= grid || (v >> 4) == (ep & 0x0fffffffu))) break;
+                        if (++polls > lim) {
+                            if (lane == 0) __hip_atomic_store(err, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            dead = true;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    same = same && __all(o >= grid || (v & 15u) == xcc_id());
+                }
+                if (lane == 0) proto[0] = !dead && same;
+            }
+            __syncthreads();
+            if (j == 0) {
+                local = proto[0] != 0u;
+                fv = 2 * ep + (local ? 1u : 0u);
+            }
+            if (j + 1 == nb) break;
+            if (w < 4) {
+                panel_quad(P[q], X, li[q], w >> 1, w & 1);
+            } else {
+                for (int e = t4; e < CB * CB / 2; e += 256)
+                    store_piece(Li + (size_t)j * CB * CB, CB, e, tile_piece(li[q], e));
+                __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+            }
+            __syncthreads();
+            if (w < 4) {
+                if (w != 1) update_quad(D[1 - q], P[q], P[q], w >> 1, w & 1);
+            } else {
+                if (w == 4 && lane == 0) {
+                    release_to(local);
+                    if (j == 0) set_flag(fD, fv);   // (for every XCD: the parts do not know the protocol yet)
+                    else set_flag_to(fD + j, fv, local);
+                }
+                for (int e = t4; e < CB * CB / 2; e += 256) store_piece(Lt(j + 1, j), n, e, tile_piece(P[q], e));
+                __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+            }
+            __syncthreads();
+        }
+        outputs(nb - 1, tid, 512);
+        store_piece(Li + (size_t)(nb - 1) * CB * CB, CB, tid, tile_piece(li[(nb - 1) & 1], tid));
     } else {
-        if (threadIdx.x == 0) wait_flag(flags + fidx(k, k), 1u, err, dead);
-        __syncthreads();
-        load_tile_d(Pb, Li + (size_t)CB * k * CB, CB);
-        __syncthreads();
-        panel_d(T, T, Pb);
-        store_tile_d(L + (size_t)CB * i * n + CB * k, Lf + (size_t)CB * i * n + CB * k, n, T, false);
+        if (tid == 0)
+            __hip_atomic_store(arr + b, ((ep & 0x0fffffffu) << 4) | xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int i, s, e;
+        owner_part64(b, nb, ow, i, s, e);
+        const bool last = e == i + 1;
+        const int jl = last ? i - 2 : e - 1;
+        const int pw = nb < ow ? nb : ow;   // (chol64_lds_bytes)
+        TileD *rt = tl, *pn = tl + pw, &in = tl[2 * pw];
+        {
+            double2 v[C64_OWMAX];
+#pragma unroll
+            for (int u = 0; u < C64_OWMAX; ++u)
+                if (s + u < e) v[u] = load_piece(G + (size_t)CB * i * ldg + (size_t)CB * (s + u), ldg, tid);
+#pragma unroll
+            for (int u = 0; u < C64_OWMAX; ++u)
+                if (s + u < e) put_piece(rt[u], tid, v[u]);
+        }
+        for (int k = s; k < e && k < i; ++k) {   // the upper triangle's tiles
+            store_piece(Lt(k, i), n, tid, zero);
+            store_piece_f(Lft(k, i), n, tid, zero);
+        }
+        for (int j = 0; j <= jl; ++j) {
+            const bool mine = j >= s;
+            if (w == 0 && (mine || j == 0)) {
+                if (j == 0) {
+                    // the call's first flag, in either protocol's value
+                    uint32_t polls = 0, got = 0;
+                    while (!dead) {
+                        got = __hip_atomic_load(fD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if ((got >> 1) == (ep & 0x7fffffffu)) break;
+                        if (++polls > lim) {
+                            if (lane == 0) __hip_atomic_store(err, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            dead = true;
+                        }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    if (lane == 0) proto[0] = dead ? 0u : got & 1u;
+                    if (dead || (got & 1u) == 0u) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                } else {
+                    wait64(lane == 0 ? fD + j : nullptr, fv, err, ep, dead, lim, local);
+                }
+            }
+            __syncthreads();
+            if (j == 0) {
+                local = proto[0] != 0u;
+                fv = 2 * ep + (local ? 1u : 0u);
+            }
+            TileD& lij = mine ? pn[j - s] : in;   // L(i, j): this part's panel, or the other part's
+            if (mine) {
+                put_piece(in, tid, load_piece_agent(Li + (size_t)j * CB * CB, CB, tid));
+                __syncthreads();
+                if (w < 4) panel_quad(lij, rt[j - s], in, w >> 1, w & 1);
+                __syncthreads();
+                const double2 v = tile_piece(lij, tid);
+                store_piece(Lt(i, j), n, tid, v);
+                __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+                __syncthreads();
+                if (tid == 0) {
+                    release_to(local);
+                    set_flag_to(fL + i * nb + j, fv, local);
+                }
+                store_piece_f(Lft(i, j), n, tid, v);
+            }
+            // the panels L(k, j) of the part's columns k < i right of j, and L(i, j) where another part forms it
+            const int k0 = std::max(s, j + 1), ke = last ? i : e, nk = ke - k0;
+            if (w == 0) {
+                const uint32_t* f = nullptr;
+                if (lane < nk) f = k0 + lane == j + 1 ? fP + j : fL + (k0 + lane) * nb + j;
+                else if (lane == nk && !mine) f = fL + i * nb + j;
+                wait64(f, fv, err, ep, dead, lim, local);
+            }
+            __syncthreads();
+            {
+                double2 v[C64_OWMAX], x = zero;
+#pragma unroll
+                for (int u = 0; u < C64_OWMAX; ++u)
+                    if (u < nk) v[u] = load_piece_agent(Lt(k0 + u, j), n, tid);
+                if (!mine) x = load_piece_agent(Lt(i, j), n, tid);
+#pragma unroll
+                for (int u = 0; u < C64_OWMAX; ++u)
+                    if (u < nk) put_piece(pn[k0 + u - s], tid, v[u]);
+                if (!mine) put_piece(in, tid, x);
+            }
+            __syncthreads();
+            for (int k = k0 + (w >> 2); k < e; k += 2) {
+                const int bi = (w >> 1) & 1, bj = w & 1;
+                if (k < i) update_quad(rt[k - s], lij, pn[k - s], bi, bj);
+                else if (bi || !bj) update_quad(rt[k - s], lij, lij, bi, bj);
+            }
+            __syncthreads();
+        }
+        if (last) {
+            store_piece(Lt(i, i - 1), n, tid, tile_piece(rt[i - 1 - s], tid));
+            store_piece(Lt(i, i), n, tid, tile_piece(rt[i - s], tid));
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+            __syncthreads();
+            if (tid == 0) {
+                release_to(local);
+                set_flag_to(fH + i, fv, local);
+            }
+        }
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     __syncthreads();
-    if (threadIdx.x == 0) publish_flag(flags + fidx(i, k), 1u);
+    if (tid == 0) cnt[b] = ep;
 }
-
-size_t chol64_lds_bytes() { return 4 * sizeof(TileD) + 2 * CB * sizeof(double); }
 
 }  // namespace
 
 struct spanqr_chol64_plan {
-    int n = 0, device = 0, nt = 0;
-    uint32_t* flags = nullptr;   // nt tile flags + the wait-error word
+    int n = 0, device = 0, nwords = 0;
+    int grid = 0, m = 1, ow = OWNER_W;    // workgroups, NXCD: all on one XCD, tiles per part
+    uint32_t* flags = nullptr;            // chol64_err_word's layout
+    std::atomic<bool> cleared{false};     // a call outside a capture has cleared the flags (later calls only count up)
 };
 
 extern "C" {
@@ -4495,15 +4720,30 @@ int spanqr_chol64_plan_create(int n, int device, spanqr_chol64_plan** out) {
     if (n < CB || n > 1024 || n % CB) return fail(SPANQR_EINVAL, "n = %d: must be a multiple of 32 in [32, 1024]", n);
     DeviceGuard dg(device);
     if (!dg.ok) return fail(SPANQR_EHIP, "cannot select HIP device %d", device);
-    const int nb = n / CB, nt = nb * (nb + 1) / 2;
-    int occ = 0, cus = 0;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)k_chol64, 256, chol64_lds_bytes()));
+    const int nb = n / CB;
+    int cus = 0, maxsh = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-    if ((long)occ * cus < nt)
-        return fail(SPANQR_EHIP, "the fp64 Cholesky needs %d resident workgroups, the device holds %d", nt, occ * cus);
+    HIPCHK(hipDeviceGetAttribute(&maxsh, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
+    HIPCHK(set_lds_limit(k_chol64, chol64_lds_bytes(1024, C64_OWMAX), maxsh));
+    // the narrowest parts that fit on one XCD, else OWNER_W spread over the device
+    int grid = 0, m = 1, ow = OWNER_W;
+    for (int v : {OWNER_W, C64_OWMAX, OWNER_W}) {
+        int occ = 0;
+        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)k_chol64, 512, chol64_lds_bytes(n, v)));
+        ow = v;
+        grid = chol64_workgroups(nb, v);
+        m = NXCD;
+        if (grid <= occ * cus / NXCD) break;
+        m = 1;
+        if (v == OWNER_W && occ * cus < grid)
+            return fail(SPANQR_EHIP, "the fp64 Cholesky needs %d resident workgroups, the device holds %d", grid,
+                        occ * cus);
+    }
     spanqr_chol64_plan* p = new spanqr_chol64_plan;
-    p->n = n; p->device = device; p->nt = nt;
-    if (hipMalloc((void**)&p->flags, (size_t)(nt + 1) * sizeof(uint32_t)) != hipSuccess) {
+    p->n = n; p->device = device;
+    p->grid = grid; p->m = m; p->ow = ow;
+    p->nwords = chol64_err_word(nb) + 1 + 2 * grid;
+    if (hipMalloc((void**)&p->flags, (size_t)p->nwords * sizeof(uint32_t)) != hipSuccess) {
         delete p;
         return fail(SPANQR_ENOMEM, "flag allocation failed");
     }
@@ -4529,8 +4769,17 @@ int spanqr_chol64(spanqr_chol64_plan* p, const double* G, long ldg, const double
     DeviceGuard dg(p->device);
     if (!dg.ok) return fail(SPANQR_EHIP, "cannot select HIP device %d", p->device);
     hipStream_t st = (hipStream_t)stream;
-    k_c64_fill<<<256, 256, 0, st>>>(p->flags, p->nt + 1, L, Lf, p->n);
-    k_chol64<<<p->nt, 256, chol64_lds_bytes(), st>>>(G, ldg, p->n, tau, L, Li, Lf, Lif, p->flags);
+    // The flags start at zero once; a captured call records the clear too (its replays then start over) but does not
+    // count as having done it.
+    if (!p->cleared.load()) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(st, &cap));
+        k_c64_clear<<<8, 256, 0, st>>>(p->flags, p->nwords);
+        HIPCHK(hipGetLastError());
+        if (cap == hipStreamCaptureStatusNone) p->cleared.store(true);
+    }
+    k_chol64<<<chol_launch_size(p->grid, 1, p->m, 0), 512, chol64_lds_bytes(p->n, p->ow), st>>>(
+        G, ldg, p->n, tau, L, Li, Lf, Lif, p->flags, p->grid, p->m, p->ow, SPIN_LIMIT);
     HIPCHK(hipGetLastError());
     return SPANQR_OK;
 }
@@ -4538,10 +4787,12 @@ int spanqr_chol64(spanqr_chol64_plan* p, const double* G, long ldg, const double
 int spanqr_chol64_status(spanqr_chol64_plan* p, void* stream) {
     if (!p) return fail(SPANQR_EINVAL, "plan is null");
     DeviceGuard dg(p->device);
-    uint32_t e = 0;
-    HIPCHK(hipMemcpyAsync(&e, p->flags + p->nt, sizeof(uint32_t), hipMemcpyDeviceToHost, (hipStream_t)stream));
+    uint32_t e[2] = {0, 0};   // the error word and workgroup 0's call counter
+    HIPCHK(hipMemcpyAsync(e, p->flags + chol64_err_word(p->n / CB), sizeof(e), hipMemcpyDeviceToHost,
+                          (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
-    if (e) return fail(SPANQR_EHIP, "fp64 Cholesky: a wait exceeded its bound (not every workgroup was resident)");
+    if (e[0] && e[0] == e[1])
+        return fail(SPANQR_EHIP, "fp64 Cholesky: a wait exceeded its bound (not every workgroup was resident)");
     return SPANQR_OK;
 }
 

@@ -73,3 +73,43 @@ def test_chol64_rejects_bad_inputs(cuda):
         kchol.chol64(torch.zeros(48, 48, device=cuda, dtype=torch.float64), 1e-9)
     with pytest.raises(ValueError):
         kchol.chol64(torch.zeros(1056, 1056, device=cuda, dtype=torch.float64), 1e-9)
+
+
+@pytest.mark.parametrize("n", [96, 192, 224, 544, 608, 640, 992])
+def test_chol64_row_parts(cuda, n):
+    """the sizes where the split changes: the first tile row with a workgroup of its own (96), rows of one and of two
+    parts (192, 224), the wider parts that still fit on one XCD (544, 608), the workgroups spread over the device
+    (640, 992), with an ill-scaled G and with a pivot row that vanishes in the last tile"""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n + 9, n)) * np.exp(rng.uniform(-6, 6, n))
+    X[:, n - 2] = X[:, 1]
+    G = X.T @ X
+    out = kchol.chol64(torch.from_numpy(G).to(cuda), 1e-10)
+    kchol.status(n, cuda)
+    for x, y, what in zip(out, oracle.chol64(G, 1e-10), ("L", "Li", "Lf", "Lif")):
+        _bits(x, y, what)
+
+
+def test_chol64_first_call_captured(cuda):
+    """a plan whose first call is captured clears its flags in the graph; eager calls and replays may then alternate"""
+    n = 288
+    rng = np.random.default_rng(1)
+    X = rng.standard_normal((n + 9, n))
+    G, t = torch.from_numpy(X.T @ X).to(cuda), torch.tensor([1e-12], device=cuda, dtype=torch.float64)
+    want = oracle.chol64(X.T @ X, 1e-12)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        kchol._plan(n, G.device)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out = kchol.chol64(G, t)
+        for k in range(4):
+            for o in out:
+                o.fill_(float("nan"))
+            g.replay()
+            eager = kchol.chol64(G, t)
+            torch.cuda.synchronize()
+            for x, e, y, what in zip(out, eager, want, ("L", "Li", "Lf", "Lif")):
+                _bits(x, y, f"{what}, replay {k}")
+                _bits(e, y, f"{what}, eager call after replay {k}")
