@@ -746,7 +746,8 @@ __device__ __forceinline__ void store16_agent(float* base, uint32_t off, uint32_
 }
 
 // the half of store_tile_op's packed layout that holds rows 16 h .. 16 h + 15, by one wavefront
-__device__ __forceinline__ void store_tile_op_half(float* dst, const Tile& src, int h, int lane, bool wt) {
+template <bool WT>
+__device__ __forceinline__ void store_tile_op_half(float* dst, const Tile& src, int h, int lane) {
     for (int u = 0; u < 2; ++u) {
         const int e = 4 * (32 * u + (lane >> 1)) + 2 * h + (lane & 1);   // e & 3 = 2 h + (0 or 1): cb = h
         const int ln = e >> 2, kk0 = 4 * (e & 1), l16 = ln & 15, lk = ln >> 4;
@@ -755,7 +756,7 @@ __device__ __forceinline__ void store_tile_op_half(float* dst, const Tile& src, 
         v.y = src[16 * h + l16][4 * (kk0 + 1) + lk];
         v.z = src[16 * h + l16][4 * (kk0 + 2) + lk];
         v.w = src[16 * h + l16][4 * (kk0 + 3) + lk];
-        if (wt) store16_agent(dst, 16u * (uint32_t)e, 4u * CB * CB, v);
+        if (WT) store16_agent(dst, 16u * (uint32_t)e, 4u * CB * CB, v);
         else *reinterpret_cast<float4*>(dst + 4 * e) = v;
     }
 }
@@ -774,8 +775,9 @@ __device__ __forceinline__ void store_tile_half(float* dst, int ld, const Tile& 
 // lane, contiguous: dst[16 lane + 8 cb + kk] = T[16 cb + (lane & 15)][4 kk + (lane >> 4)], at pair index
 // a (a + 1) / 2 + b of the packed factor (1024 floats per block).
 __device__ __forceinline__ int op_pair(int a, int b) { return a * (a + 1) / 2 + b; }
-// wt: written through the L2 (a factorisation on one XCD, whose solve runs on all of them)
-__device__ __forceinline__ void store_tile_op(float* dst, const Tile& src, int t, int nthr, bool wt) {
+// WT: written through the L2 (a factorisation on one XCD, whose solve runs on all of them)
+template <bool WT>
+__device__ __forceinline__ void store_tile_op(float* dst, const Tile& src, int t, int nthr) {
     for (int e = t; e < 256; e += nthr) {
         const int lane = e >> 2, h = e & 3, cb = h >> 1, kk0 = 4 * (h & 1), l16 = lane & 15, lk = lane >> 4;
         float4 v;
@@ -783,7 +785,7 @@ __device__ __forceinline__ void store_tile_op(float* dst, const Tile& src, int t
         v.y = src[16 * cb + l16][4 * (kk0 + 1) + lk];
         v.z = src[16 * cb + l16][4 * (kk0 + 2) + lk];
         v.w = src[16 * cb + l16][4 * (kk0 + 3) + lk];
-        if (wt) store16_agent(dst, 16u * (uint32_t)e, 4u * CB * CB, v);
+        if (WT) store16_agent(dst, 16u * (uint32_t)e, 4u * CB * CB, v);
         else *reinterpret_cast<float4*>(dst + 4 * e) = v;
     }
 }
@@ -819,9 +821,9 @@ __device__ __forceinline__ void load_tiles(Tile* dst, int n, int ld, uint32_t di
             }
 }
 
-// As load_tiles without shifts, tile q from srcf(q) with row stride ldf(q) into dstf(q), with agent-scope loads (tiles
-// that other workgroups of the launch stored)
-template <int NMAX, int NTHR, class DstF, class SrcF, class LdF>
+// As load_tiles without shifts, tile q from srcf(q) with row stride ldf(q) into dstf(q): tiles that other
+// workgroups of the launch stored (AGENT: read past the L1, which then needs no invalidation)
+template <int NMAX, int NTHR, bool AGENT, class DstF, class SrcF, class LdF>
 __device__ __forceinline__ void load_tiles_to(int n, int t, DstF dstf, SrcF srcf, LdF ldf) {
     constexpr int PER = 256 / NTHR;
     float4 v[NMAX][PER];
@@ -832,7 +834,10 @@ __device__ __forceinline__ void load_tiles_to(int n, int t, DstF dstf, SrcF srcf
             for (int u = 0; u < PER; ++u) {
                 const int e = t + u * NTHR, row = e >> 3, c4 = e & 7;
                 const uint32_t ld = (uint32_t)ldf(q);
-                v[q][u] = load16_agent(srcf(q), 4u * ((uint32_t)row * ld + 4u * (uint32_t)c4), 4u * (31u * ld + CB));
+                if (AGENT)
+                    v[q][u] = load16_agent(srcf(q), 4u * ((uint32_t)row * ld + 4u * (uint32_t)c4), 4u * (31u * ld + CB));
+                else
+                    v[q][u] = *reinterpret_cast<const float4*>(srcf(q) + (size_t)row * ld + 4 * c4);
             }
 #pragma unroll
     for (int q = 0; q < NMAX; ++q)
@@ -1370,7 +1375,10 @@ size_t chol_lds_bytes(int r, int w) {
 // congruent mod 8), and they check where they are: each owner part posts its XCD at its start, workgroup 0 compares
 // them during step 0 and says which protocol the call takes in bit 0 of every flag (the first flag an owner waits
 // for, (0, 0), is stored for all XCDs to see). What the solve reads from other XCDs, the packed operands, is then
-// written through the L2 when it is stored, so no L2 write-back is left in the kernel.
+// written through the L2 when it is stored, so no L2 write-back is left in the kernel. XCD false: a launch that is
+// spread from the start (r > 608, where the workgroups do not fit on one XCD, and r <= 160, where there is next to
+// nothing to hand over) runs without any of this: the check, the loads past the L1 and the second form of every store
+// cost it 0.4 us per launch (r <= 160) and 2 us (3001 x 736).
 static_assert(2 * chol_workgroups(CH_MAXROW, OWNER_W) <= FLAG_STRIDE - CH_MAXROW * (CH_MAXROW + 1),
               "a call counter and an arrival word per Cholesky workgroup after the panel and hand-over flags");
 
@@ -1379,7 +1387,7 @@ __device__ __forceinline__ void credit(uint32_t* colcnt, int k) {
 }
 
 // The Cholesky of workgroup b of matrix z (the pointers address matrix 0 of the launch).
-template <bool STAMP>
+template <bool STAMP, bool XCD>
 __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A, int r, const double* __restrict__ npart,
                                           int nnp, float alpha, float tau_rel, float* L, float* Li, float* Lp,
                                           uint32_t* bar, uint32_t* flags, float* scal, uint64_t* stamps, uint32_t lim,
@@ -1470,7 +1478,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
     __syncthreads();
     const uint32_t ep = calls + 1;         // this call's number (every workgroup runs every call)
     bool local = false;                    // this call's protocol (see above), known after workgroup 0's first flag
-    uint32_t fv = 0;                       // then the call's flag value: 2 ep + local
+    uint32_t fv = XCD ? 0u : 2 * ep;       // then the call's flag value: 2 ep + local
     float* pq = misc + 32;
 
     if (b == 0) {
@@ -1504,12 +1512,12 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 if (j >= 1 && j < nb - 1) credit(colcnt, j - 1);
             }
             store_tile_lower(L + o * r + o, r, z.dl[q], false, lane, 64);
-            store_tile_op(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[q], lane, 64, local);
-            if (j + 1 < nb) store_tile_op(Lp + (size_t)op_pair(j + 1, j) * CB * CB, z.P1[q], lane, 64, local);
+            store_tile_op<XCD>(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[q], lane, 64);
+            if (j + 1 < nb) store_tile_op<XCD>(Lp + (size_t)op_pair(j + 1, j) * CB * CB, z.P1[q], lane, 64);
             if (j + 2 < nb) {
                 wait_lds(p2done, (uint32_t)j + 1, err, dead, lim);   // L(j+2, j), formed by the look-ahead
                 store_tile(L + (o + 2 * CB) * r + o, r, z.P2[q], lane, 64);
-                store_tile_op(Lp + (size_t)op_pair(j + 2, j) * CB * CB, z.P2[q], lane, 64, local);
+                store_tile_op<XCD>(Lp + (size_t)op_pair(j + 2, j) * CB * CB, z.P2[q], lane, 64);
             }
         };
         // wave 3, step 0: the XCD of every owner part, once all have posted theirs
@@ -1549,7 +1557,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 if (STAMP && lane == 0) stamps[4 + 4 * j] = stamp_clock();
                 if (colcnt != nullptr && j == nb - 1) {
                     // the last column of the factor is Li_{nb-1} alone: packed, released and credited at once
-                    store_tile_op(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[p], lane, 64, local);
+                    store_tile_op<XCD>(Lp + (size_t)op_pair(j, j) * CB * CB, z.li[p], lane, 64);
                     release_to(local);
                     if (lane == 0) credit(colcnt, j);
                 }
@@ -1573,8 +1581,8 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this step's L(j+1, j) stored
             } else if (w == 3) {
                 // wave 3 publishes the previous step
-                if (j == 0) find_protocol();
-                else publish(j - 1);
+                if (j >= 1) publish(j - 1);
+                else if (XCD) find_protocol();
                 if (colcnt != nullptr && j == nb - 1 && nb >= 2) {   // column nb-2's operands, stored just now
                     release_to(local);
                     if (lane == 0) credit(colcnt, nb - 2);
@@ -1610,16 +1618,20 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                     const bool quad = !side2 || hf == 0;
                     const int qa = side2 ? 1 : hf, qb = side2 ? 0 : hf;
                     const uint32_t tb = 4u * (31u * (uint32_t)r + CB);   // bytes of a tile's rows
+                    auto fetch16 = [&](const float* b0, uint32_t o, uint32_t bytes) {
+                        if (XCD) return load16_agent(b0, o, bytes);
+                        return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(b0) + o);
+                    };
                     float4 v[5];
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const int e = lane + 64 * u, row = 16 * hf + (e >> 3), c4 = e & 7;
                         const uint32_t off = 4u * ((uint32_t)row * (uint32_t)r + 4u * (uint32_t)c4);
-                        v[u] = load16_agent(s0, off, tb);
-                        v[2 + u] = load16_agent(s1, off, tb);
+                        v[u] = fetch16(s0, off, tb);
+                        v[2 + u] = fetch16(s1, off, tb);
                     }
                     const int qrow = 16 * qa + (lane >> 2), qc4 = 4 * qb + (lane & 3);
-                    if (quad) v[4] = load16_agent(s3, 4u * ((uint32_t)qrow * (uint32_t)r + 4u * (uint32_t)qc4), tb);
+                    if (quad) v[4] = fetch16(s3, 4u * ((uint32_t)qrow * (uint32_t)r + 4u * (uint32_t)qc4), tb);
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const int e = lane + 64 * u, row = 16 * hf + (e >> 3), c4 = e & 7;
@@ -1646,7 +1658,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                         // its half for the output and the later kernels (the owners form their own copy)
                         const size_t o = (size_t)CB * (j - 1);
                         store_tile_half(L + (o + 3 * CB) * r + o, r, z.C2[p], hf, lane);
-                        store_tile_op_half(Lp + (size_t)op_pair(j + 2, j - 1) * CB * CB, z.C2[p], hf, lane, local);
+                        store_tile_op_half<XCD>(Lp + (size_t)op_pair(j + 2, j - 1) * CB * CB, z.C2[p], hf, lane);
                     } else if (j >= 2) {                                               // T(j+2, j+1), block j-2
                         if (hf) update32_wave_q<0xC>(R2[2], R2[2], R2[4], z.C2[pp]);
                         else update32_wave_q<0x3>(R2[2], R2[2], R2[4], z.C2[pp]);
@@ -1678,11 +1690,11 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                     }
                 }
                 // T(j+2, j) and the packed L(j+2, j-1) are stored (in agent mode wave 3's release covers them)
-                if (!side2) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+                if (XCD && !side2) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
                 if (STAMP && w == 1 && lane == 0) stamps[2 + 4 * nb + j] = stamp_clock();
             }
             __syncthreads();
-            if (j == 0) {
+            if (XCD && j == 0) {
                 local = reinterpret_cast<uint32_t*>(misc)[3] != 0u;
                 fv = 2 * ep + (local ? 1u : 0u);
             }
@@ -1694,7 +1706,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
         if (w == 3) publish(nb - 1);
         if (STAMP && tid == 0) stamps[1 + 4 * nb] = stamp_clock();
     } else {
-        if (tid == 0) set_flag(arr + b, (ep << 4) | xcc_id());
+        if (XCD && tid == 0) set_flag(arr + b, (ep << 4) | xcc_id());
         // Owner part: tile row i, tiles T(i, s..e-1) in LDS. rt[k - s] = T(i, k); pn[k - s] = L(k, j) of the current
         // column block for the part's columns k < i; li = Li_j; pin = L(i, j) when another part of the row holds
         // T(i, j). Each part runs blocks j until its tiles are done: the last part (which holds T(i, i)) to block
@@ -1737,7 +1749,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 } else if (lane == nk + 1 && !mine && j >= 1) {
                     f = flagL + i * nb + j;
                 }
-                if (j == 0) {
+                if (XCD && j == 0) {
                     // the call's first flag, (0, 0) alone, in either protocol's value
                     uint32_t polls = 0, got = 0;
                     while (!dead) {
@@ -1756,7 +1768,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 }
             }
             __syncthreads();
-            if (j == 0) {
+            if (XCD && j == 0) {
                 local = reinterpret_cast<uint32_t*>(misc)[3] != 0u;
                 fv = 2 * ep + (local ? 1u : 0u);
             }
@@ -1764,7 +1776,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
             if (bst) bs[0] = stamp_clock();
             // one batch: Li_j; per column k, the finished L(j+1, j) or T(k, j) through block j-1; T(i, j) into pin
             if (q4)
-                load_tiles_to<OWNER_WMAX + 2, 256>(1 + nk + (mine ? 0 : 1), tid,
+                load_tiles_to<OWNER_WMAX + 2, 256, XCD>(1 + nk + (mine ? 0 : 1), tid,
                                                 [&](int q) -> Tile& { return q == 0 ? li : q <= nk ? pn[k0 + q - 1 - s] : pin; },
                                                 [&](int q) {
                                                     if (q == 0) return (const float*)(Li + (size_t)CB * j * CB);
@@ -1786,7 +1798,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
             if (mine) {
                 // L(i, j): the output, and its packed form for the solve (released below, with the column credit)
                 if (q4) store_tile(L + (size_t)CB * i * r + (size_t)CB * j, r, lij);
-                else store_tile_op(Lp + (size_t)op_pair(i, j) * CB * CB, lij, tid - 256, 256, local);
+                else store_tile_op<XCD>(Lp + (size_t)op_pair(i, j) * CB * CB, lij, tid - 256, 256);
             } else if (hand && q4) {
                 // workgroup 0 reads L(i, i-4) with the handed-over row: this part's own copy (the same bits as the
                 // holder's), stored before the hand-over
@@ -1891,6 +1903,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
 // m = 1 its workgroups are spread over the XCDs. An index that is no Cholesky workgroup (a gap of a last group of
 // fewer than m matrices, or past them all) gets its rank among such indices in `other`.
 constexpr int NXCD = 8;
+constexpr int XCD_MIN_R = 160;   // up to two owner parts: spread, 1024 x 160 141.8 us per call, on one XCD 143.7 (192: 153.2, 150.8)
 static_assert(NXCD == 8, "chol_role's shift");
 // (Divisions only where a launch has more than one group of matrices: at the head of every workgroup they cost ~1 us.)
 __device__ __forceinline__ int chol_role(int idx, int grid, int nz, int m, int& z, int& other) {
@@ -1919,7 +1932,7 @@ int chol_launch_size(int grid, int nz, int m, int others) {
 
 // tau_ptr (nnp == 0 only; may be null): the absolute pivot floor read from device memory instead of tau_rel (chol32
 // with tau as a device tensor, kchol.py:24-28: no host synchronisation)
-template <bool STAMP>
+template <bool STAMP, bool XCD>
 __global__ __launch_bounds__(512) void k_chol(float* A, int r, const double* __restrict__ npart, int nnp, float alpha,
                                               float tau_rel, float* L, float* Li, float* Lp, uint32_t* bar,
                                               uint32_t* flags, float* scal, uint64_t* stamps, uint32_t lim, int ow,
@@ -1927,7 +1940,7 @@ __global__ __launch_bounds__(512) void k_chol(float* A, int r, const double* __r
     int z = 0, other = 0;
     const int b = chol_role(blockIdx.x, grid, nz, m, z, other);
     if (b < 0) return;
-    chol_body<STAMP>(b, z, A, r, npart, nnp, alpha, tau_rel, L, Li, Lp, bar, flags, scal, stamps, lim, nullptr, ow, grid,
+    chol_body<STAMP, XCD>(b, z, A, r, npart, nnp, alpha, tau_rel, L, Li, Lp, bar, flags, scal, stamps, lim, nullptr, ow, grid,
                      tau_ptr);
 }
 
@@ -2332,12 +2345,12 @@ struct SolveArgs {
 
 // Q > 0: the solve of k_trsm (Q column blocks per wave, RB row blocks of 16 per workgroup); Q = 0: trsm_wave_body
 // with NBC = RB column blocks (eight row blocks per workgroup).
-template <bool PASS1, int Q, int RB>
+template <bool PASS1, int Q, int RB, bool XCD>
 __global__ __launch_bounds__(64 * TRSM_NW) void k_chol_solve(const CholArgs c, const SolveArgs t) {
     int z = 0, b = 0;
     const int cb = chol_role(blockIdx.x, c.grid, c.nz, c.m, z, b);
     if (cb >= 0) {
-        chol_body<false>(cb, z, c.A, c.r, c.npart, c.nnp, c.alpha, c.tau_rel, c.L, c.Li, c.Lp, c.bar, c.flags, c.scal,
+        chol_body<false, XCD>(cb, z, c.A, c.r, c.npart, c.nnp, c.alpha, c.tau_rel, c.L, c.Li, c.Lp, c.bar, c.flags, c.scal,
                          nullptr, c.lim, c.colcnt, c.ow, c.grid);
         return;
     }
@@ -3061,12 +3074,11 @@ int launch_chol(spanqr_plan* p, float alpha, float tau, float* scal, hipStream_t
         uint32_t* flags = p->flags + (size_t)z0 * FLAG_STRIDE;
         float* sc = scal ? scal + (size_t)z0 * SCAL_STRIDE : nullptr;
         const dim3 grid(chol_launch_size(p->chol_grid, nz, p->chol_m, 0));
-        if (stamp)
-            k_chol<true><<<grid, 512, lds, st>>>(A, p->r, np, nnp, alpha, tau, L, Li, Lp, bar, flags, sc, p->stamps,
-                                                 g_spin_limit, p->owner_w, p->chol_grid, nz, p->chol_m, tau_ptr);
-        else
-            k_chol<false><<<grid, 512, lds, st>>>(A, p->r, np, nnp, alpha, tau, L, Li, Lp, bar, flags, sc, p->stamps,
-                                                  g_spin_limit, p->owner_w, p->chol_grid, nz, p->chol_m, tau_ptr);
+        const bool xcd = p->chol_m == NXCD;
+        auto* kernel = stamp ? (xcd ? k_chol<true, true> : k_chol<true, false>)
+                             : (xcd ? k_chol<false, true> : k_chol<false, false>);
+        kernel<<<grid, 512, lds, st>>>(A, p->r, np, nnp, alpha, tau, L, Li, Lp, bar, flags, sc, p->stamps, g_spin_limit,
+                                       p->owner_w, p->chol_grid, nz, p->chol_m, tau_ptr);
         HIPCHK(hipGetLastError());
     }
     return SPANQR_OK;
@@ -3102,12 +3114,25 @@ hipError_t trsm_limits(int maxsh) {
 
 // the fused instantiations: Q = 1 (r <= 256) with one row block, Q = 2 (r <= 512) with one or two, Q = 4
 // (r <= 1024) with one, and the wavefront-per-row-block solve (Q = 0) for r/32 = RB = 2, 4, 6, 8 column blocks
+// The hand-over protocols each is built for: the one for a single XCD (which also runs spread, as a batch may need it
+// at r = 192..512) and the one without it, for the widths where plans spread the factorisation.
+enum { FUSED_SPREAD = 1, FUSED_XCD = 2 };
+constexpr int fused_protocols(int q, int rb) {
+    return q == 0 ? (rb >= 6 ? FUSED_XCD : FUSED_SPREAD) : q == 2 ? FUSED_XCD : FUSED_SPREAD | FUSED_XCD;
+}
 template <int Q, int RB>
 hipError_t fused_limits(int maxsh) {
     const int rmax = Q > 0 ? trsm_q_max_r(Q) : RB * CB;
     const size_t need = fused_lds(rmax, OWNER_WMAX, Q, RB);
-    hipError_t e = set_lds_limit(k_chol_solve<true, Q, RB>, need, maxsh);
-    if (e == hipSuccess) e = set_lds_limit(k_chol_solve<false, Q, RB>, need, maxsh);
+    hipError_t e = hipSuccess;
+    if constexpr ((fused_protocols(Q, RB) & FUSED_XCD) != 0) {
+        if (e == hipSuccess) e = set_lds_limit(k_chol_solve<true, Q, RB, true>, need, maxsh);
+        if (e == hipSuccess) e = set_lds_limit(k_chol_solve<false, Q, RB, true>, need, maxsh);
+    }
+    if constexpr ((fused_protocols(Q, RB) & FUSED_SPREAD) != 0) {
+        if (e == hipSuccess) e = set_lds_limit(k_chol_solve<true, Q, RB, false>, need, maxsh);
+        if (e == hipSuccess) e = set_lds_limit(k_chol_solve<false, Q, RB, false>, need, maxsh);
+    }
     return e;
 }
 
@@ -3133,8 +3158,8 @@ int kernel_lds_limits(int device) {
     if (e == hipSuccess) e = fused_limits<0, 4>(maxsh);
     if (e == hipSuccess) e = fused_limits<0, 6>(maxsh);
     if (e == hipSuccess) e = fused_limits<0, 8>(maxsh);
-    if (e == hipSuccess) e = set_lds_limit(k_chol<true>, chol_lds_bytes(KCH_MAX_R, OWNER_WMAX), maxsh);
-    if (e == hipSuccess) e = set_lds_limit(k_chol<false>, chol_lds_bytes(KCH_MAX_R, OWNER_WMAX), maxsh);
+    for (auto* k : {k_chol<true, true>, k_chol<true, false>, k_chol<false, true>, k_chol<false, false>})
+        if (e == hipSuccess) e = set_lds_limit(k, chol_lds_bytes(KCH_MAX_R, OWNER_WMAX), maxsh);
     if (e == hipSuccess) e = set_lds_limit(k_nsapply_res<512>, nsr_lds_bytes<512>(), maxsh);
     if (e != hipSuccess) return fail(SPANQR_EHIP, "setting the kernels' LDS limits failed: %s", hipGetErrorString(e));
     if (track) g_lds_done[device] = true;
@@ -3201,7 +3226,15 @@ void launch_trsm(const spanqr_plan* p, const MatsIn& A, long lda, bool pass1, fl
 
 template <bool PASS1, int Q, int RB>
 void launch_fused_t(dim3 grid, size_t lds, hipStream_t st, const CholArgs& c, const SolveArgs& t) {
-    k_chol_solve<PASS1, Q, RB><<<grid, 64 * TRSM_NW, lds, st>>>(c, t);
+    constexpr int pr = fused_protocols(Q, RB);
+    if constexpr (pr == FUSED_XCD) {
+        k_chol_solve<PASS1, Q, RB, true><<<grid, 64 * TRSM_NW, lds, st>>>(c, t);
+    } else if constexpr (pr == FUSED_SPREAD) {
+        k_chol_solve<PASS1, Q, RB, false><<<grid, 64 * TRSM_NW, lds, st>>>(c, t);
+    } else {
+        if (c.m == NXCD) k_chol_solve<PASS1, Q, RB, true><<<grid, 64 * TRSM_NW, lds, st>>>(c, t);
+        else k_chol_solve<PASS1, Q, RB, false><<<grid, 64 * TRSM_NW, lds, st>>>(c, t);
+    }
 }
 
 template <bool PASS1>
@@ -3455,8 +3488,8 @@ int plan_device_setup(spanqr_plan* p, int device) {
     int cus = 0;
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     p->cus = cus;
-    // The owner part width and the placement. A factorisation whose workgroups all fit on one XCD goes there (m =
-    // NXCD); otherwise its workgroups are spread (m = 1). One matrix takes the narrowest parts, in tiles, that fit on
+    // The owner part width and the placement. A factorisation wider than XCD_MIN_R whose workgroups all fit on one XCD
+    // goes there (m = NXCD); otherwise its workgroups are spread (m = 1). One matrix takes the narrowest parts, in tiles, that fit on
     // one XCD with at most 8 tiles (12-tile parts there: 671 us per call at 3001 x 736, 6-tile parts spread: 656), or
     // else OWNER_W; a batch the narrowest parts that run its Cholesky in the fewest launches. Each launch
     // needs all its workgroups resident at once: several matrices take at most 7/8 of an XCD or three quarters of the
@@ -3467,11 +3500,11 @@ int plan_device_setup(spanqr_plan* p, int device) {
         for (int pass = 0; pass < 2; ++pass)
             for (int w : widths) {
                 int o = 0;
-                HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (const void*)k_chol<true>, 512, chol_lds_bytes(r, w)));
+                HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (const void*)k_chol<true, true>, 512, chol_lds_bytes(r, w)));
                 const int grid = chol_workgroups(r / CB, w), xcd = o * cus / NXCD;
                 int bmax;
                 if (pass == 0) {
-                    if (grid > xcd || (p->batch == 1 && w > 8)) continue;
+                    if (r <= XCD_MIN_R || grid > xcd || (p->batch == 1 && w > 8)) continue;
                     bmax = NXCD * std::max(1, xcd * 7 / 8 / grid);
                 } else {
                     if (p->batch == 1 && best_n == 1) break;
