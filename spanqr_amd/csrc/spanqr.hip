@@ -166,15 +166,23 @@ __device__ __forceinline__ float rsqrt_sw(float x) {
 // ---------------------------------------------------------------------------------------------------------------
 // max|x| partials (torch.linalg.vector_norm(X, inf), kcholqr.py:102): the largest bit pattern of |x| per workgroup;
 // NaN patterns sort above +inf, so NaN propagates as in torch. As the first kernel of a call it also clears the
-// matrix's wait-error word (bar[2], set by a bounded wait of this call's Cholesky that gave up).
+// matrix's wait-error word (bar[2], set by a bounded wait of this call's Cholesky that gave up). The column-blocked path
+// runs kcholf once or twice per block: its first kernel (BLK_START) clears the whole call's error word bar[3] too, and
+// each kcholf keeps the error of the one before it there (BLK_KEEP), so the call's error is bar[2] or bar[3].
 // ---------------------------------------------------------------------------------------------------------------
+constexpr int BLK_START = 1, BLK_KEEP = 2;
 template <int NT>
 __global__ __launch_bounds__(NT) void k_amax(const MatsIn Xs, long ldx, int K, int r, uint32_t* __restrict__ part,
-                                              uint32_t* bar = nullptr) {
+                                              uint32_t* bar = nullptr, int blocked = 0) {
     // the maximum is exact in any order, so the block size (and with it the order) leaves the result unchanged
     const float* __restrict__ X = Xs.p[blockIdx.z];
     part += (size_t)blockIdx.z * AMAX_BLOCKS;
-    if (bar != nullptr && blockIdx.x == 0 && threadIdx.x == 0) bar[(size_t)blockIdx.z * BAR_STRIDE + 2] = 0u;
+    if (bar != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+        uint32_t* b = bar + (size_t)blockIdx.z * BAR_STRIDE;
+        if (blocked == BLK_START) b[3] = 0u;
+        else if (blocked == BLK_KEEP && b[2] != 0u) b[3] = 1u;
+        b[2] = 0u;
+    }
     uint32_t m = 0;
     const int r4 = r >> 2;
     const int n4 = K * r4;
@@ -366,30 +374,59 @@ __global__ __launch_bounds__(512) void k_gram(const MatsIn As, long lda, int K, 
 // the tile entries (32 qi + 2 m + a, 32 qj + 2 n + b) -- each element's chain still runs over the split's rows in
 // order, four per MFMA. A buffer resource per chunk and strip whose range ends at the split's last row makes rows
 // past it read as 0; a strip past the columns rc (r % 64 == 32) has an empty range. GR_DEPTH chunks are in flight
-// per wavefront.
+// per wavefront. CROSS: the partials of A^T B (k_gram's CROSS), with workgroups of four wavefronts or of one (64
+// threads, 4 U workgroups per split: the quadrants of U tiles, eight tiles at a time).
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int GR_DEPTH = 3;   // chunks in flight per wavefront (16 loads each; vmcnt counts at most 63 outstanding)
+template <bool CROSS>
 __global__ __launch_bounds__(256) void k_gramr(const MatsIn As, long lda, int K, int nt, int KS, float* __restrict__ P,
-                                               int rc) {
-    const int u = blockIdx.x, sp = blockIdx.y, U = gridDim.x;
+                                               int rc, const float* __restrict__ Bx = nullptr, long ldbx = 0,
+                                               int ntb = 0, int rcbx = 0) {
+    const int sp = blockIdx.y, tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+    int u, w, U, ti, tj;
+    if (CROSS && blockDim.x == 64) {
+        // one wavefront per workgroup: quadrants 8 apart, so that a tile's four share an XCD
+        U = gridDim.x >> 2;
+        const int full = U & ~7, x = blockIdx.x;
+        if (x < 4 * full) {
+            u = (x >> 5) * 8 + (x & 7);
+            w = (x >> 3) & 3;
+        } else {
+            u = full + ((x - 4 * full) >> 2);
+            w = x & 3;
+        }
+    } else {
+        U = gridDim.x;
+        u = blockIdx.x;
+        w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    }
     const float* __restrict__ A = As.p[blockIdx.z];
+    const float* __restrict__ B = CROSS ? Bx : A;
+    const long ldb = CROSS ? ldbx : lda;
+    const int rcb = CROSS ? rcbx : rc;
     P += (size_t)blockIdx.z * gridDim.y * U * TB * TB;
-    int ti, tj;
-    upper_tile(u, nt, ti, tj);
-    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int qi = w >> 1, qj = w & 1, l16 = lane & 15, lk = lane >> 4;
+    if (CROSS) {
+        ti = u / ntb;
+        tj = u - ti * ntb;
+    } else {
+        upper_tile(u, nt, ti, tj);
+    }
+    const int qi = w >> 1, qj = w & 1;
     const int ca = ti * TB + 32 * qi, cb = tj * TB + 32 * qj;   // the block's first column in each strip
     const int k0 = sp * KS, k1 = (k0 + KS < K) ? k0 + KS : K;
     const int nch = k1 > k0 ? (k1 - k0 + BK - 1) / BK : 0;
     const char* baseA = reinterpret_cast<const char*>(A + ca);
-    const char* baseB = reinterpret_cast<const char*>(A + cb);
-    uint32_t off[BK / 4];   // lda < 2^24 (checked by the host): 32 rows of bytes fit 31 bits
+    const char* baseB = reinterpret_cast<const char*>(B + cb);
+    uint32_t off[BK / 4], offb[BK / 4];   // lda, ldb < 2^24 (checked by the host): 32 rows of bytes fit 31 bits
 #pragma unroll
-    for (int kk = 0; kk < BK / 4; ++kk) off[kk] = ((uint32_t)(4 * kk + lk) * (uint32_t)lda + 2u * (uint32_t)l16) * 4u;
+    for (int kk = 0; kk < BK / 4; ++kk) {
+        off[kk] = ((uint32_t)(4 * kk + lk) * (uint32_t)lda + 2u * (uint32_t)l16) * 4u;
+        offb[kk] = CROSS ? ((uint32_t)(4 * kk + lk) * (uint32_t)ldb + 2u * (uint32_t)l16) * 4u : off[kk];
+    }
     const int last = nch > 0 ? nch - 1 : 0;
     // bytes per row of each strip's range (0: the strip is past rc and reads as 0)
     const int rowa = __builtin_amdgcn_readfirstlane(ca < rc ? (int)lda * 4 : 0);
-    const int rowbb = __builtin_amdgcn_readfirstlane(cb < rc ? (int)lda * 4 : 0);
+    const int rowbb = __builtin_amdgcn_readfirstlane(cb < rcb ? (int)ldb * 4 : 0);
     // slot d holds chunk c with c % GR_DEPTH == d; a chunk past the split's last reads that one again (unused)
     float ra[GR_DEPTH][BK / 4][2], rb[GR_DEPTH][BK / 4][2];
     auto gload = [&](int c, float (*xa)[2], float (*xb)[2]) {
@@ -399,14 +436,15 @@ __global__ __launch_bounds__(256) void k_gramr(const MatsIn As, long lda, int K,
         const int numa = __builtin_amdgcn_readfirstlane(nv * rowa);
         const int numb = __builtin_amdgcn_readfirstlane(nv * rowbb);
         const size_t rowb = (size_t)(kr < K ? kr : 0) * (size_t)lda * 4;
+        const size_t rowb2 = CROSS ? (size_t)(kr < K ? kr : 0) * (size_t)ldb * 4 : rowb;
         const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(baseA + rowb), (short)0, numa,
                                                                             BUF_RSRC_WORD3);
-        const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(baseB + rowb), (short)0, numb,
+        const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(baseB + rowb2), (short)0, numb,
                                                                             BUF_RSRC_WORD3);
 #pragma unroll
         for (int kk = 0; kk < BK / 4; ++kk) {
             const auto va = __builtin_amdgcn_raw_buffer_load_b64(rA, (int)off[kk], 0, 0);
-            const auto vb = __builtin_amdgcn_raw_buffer_load_b64(rB, (int)off[kk], 0, 0);
+            const auto vb = __builtin_amdgcn_raw_buffer_load_b64(rB, (int)offb[kk], 0, 0);
             xa[kk][0] = __uint_as_float(va[0]);
             xa[kk][1] = __uint_as_float(va[1]);
             xb[kk][0] = __uint_as_float(vb[0]);
@@ -2790,22 +2828,17 @@ __global__ __launch_bounds__(256, 2) void k_nsapply_res(const MatsIn Ys, long ld
 // at 17408x256, 9.8 -> 5.5 at 32768x256), 256 below (0.1 us faster at 768x512 and 2048x256); AMAX_BLOCKS
 // partial maxima either way
 constexpr long AMAX_BIG = 1L << 20;
-void launch_amax(const MatsIn& X, long ldx, int K, int r, uint32_t* part, uint32_t* bar, int n, hipStream_t st) {
+void launch_amax(const MatsIn& X, long ldx, int K, int r, uint32_t* part, uint32_t* bar, int n, hipStream_t st,
+                 int blocked = 0) {
     if ((long)K * r >= AMAX_BIG)
-        k_amax<1024><<<dim3(AMAX_BLOCKS, 1, n), 1024, 0, st>>>(X, ldx, K, r, part, bar);
+        k_amax<1024><<<dim3(AMAX_BLOCKS, 1, n), 1024, 0, st>>>(X, ldx, K, r, part, bar, blocked);
     else
-        k_amax<256><<<dim3(AMAX_BLOCKS, 1, n), 256, 0, st>>>(X, ldx, K, r, part, bar);
+        k_amax<256><<<dim3(AMAX_BLOCKS, 1, n), 256, 0, st>>>(X, ldx, K, r, part, bar, blocked);
 }
 
 // word[i * stride] = 0 for i < n (clears wait-error words where no k_amax runs first)
 __global__ void k_clear_words(uint32_t* word, int n, int stride) {
     if ((int)threadIdx.x < n) word[(size_t)threadIdx.x * stride] = 0u;
-}
-
-// bar[3] |= bar[2]: the column-blocked path runs kcholf once per block, each run clearing bar[2] first, so the
-// error of the whole call is kept in bar[3] (cleared at the call's start)
-__global__ void k_keep_error(uint32_t* bar) {
-    if (threadIdx.x == 0 && bar[2] != 0u) bar[3] = 1u;
 }
 
 // Q = Y for a call without polish steps (ns = 0), NaN when the call's Cholesky gave up a wait (as k_nsapply)
@@ -3011,7 +3044,7 @@ void launch_gram_n(const spanqr_plan* p, const MatsIn& A, long lda, dim3 grid, b
 void launch_gram(const spanqr_plan* p, const MatsIn& A, long lda, int n, bool scale, bool kahan, hipStream_t st) {
     const dim3 grid(p->U, p->S, n);
     if (!kahan && !scale && p->KS >= GRAMR_MIN_KS)
-        k_gramr<<<grid, 256, 0, st>>>(A, lda, p->K, p->nt, p->KS, p->P, p->r);
+        k_gramr<false><<<grid, 256, 0, st>>>(A, lda, p->K, p->nt, p->KS, p->P, p->r);
     else if (p->KS <= GRAM_DEEP_KS)
         launch_gram_n<2>(p, A, lda, grid, scale, kahan, st);
     else
@@ -3347,7 +3380,8 @@ void launch_nsapply(const spanqr_plan* p, const MatsIn& Y, long ldy, const MatsO
 // every kernel (profiling).
 int enqueue_orth(spanqr_plan* p, int n, const MatsIn& X, long ldx, const MatsOut& Q, long ldq, float eps, float alpha,
                  float tau, int ns, hipStream_t st, bool rec, Dust dz = Dust{nullptr, 0}) {
-    if (dz.z == nullptr) dz = Dust{p->Z, p->r};
+    const bool blocked = dz.z != nullptr;
+    if (!blocked) dz = Dust{p->Z, p->r};
     p->last_n = n;
     int rc;
     auto mark = [&]() -> int {
@@ -3357,7 +3391,8 @@ int enqueue_orth(spanqr_plan* p, int n, const MatsIn& X, long ldx, const MatsOut
         }
         return SPANQR_OK;
     };
-    launch_amax(X, ldx, p->K, p->r, p->amax_part, p->bar, n, st);
+    // (dust from outside the plan: one kcholf of the column-blocked path)
+    launch_amax(X, ldx, p->K, p->r, p->amax_part, p->bar, n, st, blocked ? BLK_KEEP : 0);
     if ((rc = mark())) return rc;
     const MatsIn bin[2] = {buf_in(p, p->Y0), buf_in(p, p->Y1)};
     const MatsOut bout[2] = {buf_out(p, p->Y0), buf_out(p, p->Y1)};
@@ -3667,7 +3702,16 @@ void project(const spanqr_plan* p, const float* Q, long ldq, int j, const float*
     int S = 0, KS = 0;
     split_policy(p->K, U, &S, &KS);
     const MatsIn P = mats_in(&Q, 1);
-    if (KS <= GRAM_DEEP_KS)
+    if (KS >= GRAMR_MIN_KS) {
+        // A workgroup per tile, or per quadrant where whole tiles would load the CUs unevenly (by more than a quarter):
+        // at K = 17408, 256 columns, us per launch, tiles / quadrants: j = 256 25 / 30, 512 45 / 54, 1024 86 / 103 (512
+        // tiles and splits on 256 CUs: even), 768 82 / 79 (528), 1280 135 / 122 (560), 1536 152 / 142 (576), 1792 184 /
+        // 168 (560). k_gram, for all of them: 26, 49, 94, 91, 146, 170, 202.
+        const long cus = p->blk->cus, wgs = (long)U * S;
+        const bool quads = (wgs + cus - 1) / cus * cus * 4 > wgs * 5;
+        k_gramr<true><<<dim3(quads ? 4 * U : U, S), quads ? 64 : 256, 0, st>>>(P, ldq, p->K, 0, KS, p->Tp, j, Cin, ldc,
+                                                                            ntb, BW);
+    } else if (KS <= GRAM_DEEP_KS)
         k_gram<false, false, true, 2><<<dim3(U, S), 512, 0, st>>>(P, ldq, p->K, 0, KS, p->bamax, p->Tp, Cin, ldc, ntb,
                                                                  j, BW);
     else
@@ -3690,8 +3734,7 @@ int enqueue_borth(spanqr_plan* p, const float* X, long ldx, float* Q, long ldq, 
                   int ns, hipStream_t st) {
     const int K = p->K, BW = p->bw;
     p->last_n = 1;
-    k_clear_words<<<1, 64, 0, st>>>(p->blk->bar + 3, 1, BAR_STRIDE);
-    launch_amax(mats_in(&X, 1), ldx, K, p->r, p->bamax, nullptr, 1, st);
+    launch_amax(mats_in(&X, 1), ldx, K, p->r, p->bamax, p->blk->bar, 1, st, BLK_START);
     const int sgrid = (K * (BW / 4) + 255) / 256 < 1024 ? (K * (BW / 4) + 255) / 256 : 1024;
     int rc;
     for (int jb = 0; jb < p->nblk; ++jb) {
@@ -3707,13 +3750,11 @@ int enqueue_borth(spanqr_plan* p, const float* X, long ldx, float* Q, long ldq, 
         if ((rc = enqueue_orth(p->blk, 1, mats_in(&Wc, 1), BW, mats_out(&Qj, 1), ldq, eps, alpha, tau, ns, st, false,
                                dz)))
             return rc;
-        k_keep_error<<<1, 64, 0, st>>>(p->blk->bar);
         if (j > 0 && p->reorth) {
             project(p, Q, ldq, j, Qj, ldq, p->W, st);
             if ((rc = enqueue_orth(p->blk, 1, mats_in(&Wc, 1), BW, mats_out(&Qj, 1), ldq, eps, alpha, tau, ns, st,
                                    false, dz)))
                 return rc;
-            k_keep_error<<<1, 64, 0, st>>>(p->blk->bar);
         }
     }
     HIPCHK(hipGetLastError());
@@ -4093,13 +4134,13 @@ int spanqr_plan_status(spanqr_plan* p, void* stream) {
     if (!dg.ok) return fail(SPANQR_EHIP, "cannot select HIP device %d", p->device);
     const spanqr_plan* q = p->blk ? p->blk : p;
     const int n = p->blk ? 1 : (p->last_n < 1 ? 1 : p->last_n);
-    const int word = p->blk ? 3 : 2;   // the column-blocked path keeps the whole call's error in word 3
     uint32_t w[SPANQR_MAX_BATCH * BAR_STRIDE];
     HIPCHK(hipMemcpyAsync(w, q->bar, (size_t)n * BAR_STRIDE * sizeof(uint32_t), hipMemcpyDeviceToHost,
                           (hipStream_t)stream));
     HIPCHK(hipStreamSynchronize((hipStream_t)stream));
     for (int i = 0; i < n; ++i)
-        if (w[(size_t)i * BAR_STRIDE + word] != 0u)
+        // (word 3: an earlier block's, on the column-blocked path)
+        if (w[(size_t)i * BAR_STRIDE + 2] != 0u || (p->blk && w[(size_t)i * BAR_STRIDE + 3] != 0u))
             return fail(SPANQR_EHIP, "matrix %d of the last call: a bounded wait of its Cholesky gave up (not every "
                                      "workgroup of the launch was resident); its Q is NaN", i);
     return SPANQR_OK;

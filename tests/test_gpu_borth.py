@@ -154,3 +154,17 @@ def test_blocked_plan_refused_where_it_does_not_apply(cuda):
     assert b"column-blocked" in L.spanqr_last_error()
     assert L.spanqr_orth_f32(plan.handle, X.data_ptr(), 512, X.data_ptr(), r, 5e-7, 1e-7, 1e-8, 2,
                              stream_handle(cuda)) == -1
+
+
+@pytest.mark.parametrize("K,r,b", [(2501, 1024, 512),     # splits of 320 rows, a workgroup per tile
+                                   (2301, 1088, 544),     # 81 tiles in 7 splits: a workgroup per quadrant, half tiles
+                                   (3521, 960, 320)])     # 25 tiles (short splits), then 50 in 11: quadrants
+def test_borth_long_splits(cuda, K, r, b):
+    """projections whose splits are long enough for the register-fed product, in both of its workgroup forms, with a
+    ragged last split, half-used last tiles and an X with a wider row stride"""
+    g = torch.Generator().manual_seed(K)
+    wide = torch.randn(K, r + 8, generator=g)
+    X = wide[:, 4:4 + r]
+    print(f"borth long splits {K}x{r} b={b}", flush=True)
+    Q = borth(wide.to(cuda)[:, 4:4 + r], b=b)
+    assert_bits(Q, oracle.borth(X.contiguous().numpy(), b), f"borth {K}x{r} b={b}")
