@@ -1104,10 +1104,6 @@ __device__ __forceinline__ void release() {
 __device__ __forceinline__ void set_flag(uint32_t* f, uint32_t ep) {
     __hip_atomic_store(f, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void publish_flag(uint32_t* f, uint32_t ep) {
-    release();
-    set_flag(f, ep);
-}
 // The same between workgroups that share an XCD's L2 (local): the stores are complete -- in that L2 -- once vmcnt says
 // so, and the flag is stored there too (the agent-scope polls read past the CUs' L1 and find it in the L2). Other
 // XCDs see neither until the kernel ends, so a flag that workgroups elsewhere may be polling is set with set_flag.
@@ -4359,6 +4355,9 @@ int spanqr_orth_f32_noalloc(int K, int r, const float* X, long ldx, float* Q, lo
 // one CU, and beside it the loop through row j+2's part (Li_j, panel, update, hand-over), so the workgroups of a
 // factorisation sit on one XCD where they fit and hand over through its L2 (n <= 608; the protocol of the fp32
 // factorisation, with the same check of where the workgroups are).
+// Measured, us per call, before (a workgroup per tile, scalar fma products, hand-overs across XCDs, a launch to clear the
+// flags) and now: n = 32 59.6 / 22.1, 256 476 / 100, 512 957 / 193, 1024 (spread) 1980 / 423; ~12 us per 32 columns, of
+// which the tile factor is ~7.
 // Publication: stores, wait for them, release, a flag that carries the call number; waits are bounded and the error
 // word takes the call number of a call in which one gave up. Rows wait only on earlier rows' same block and on
 // workgroup 0, which waits only on the row before the one it factors, so with every workgroup resident (checked when
