@@ -17,6 +17,13 @@
  *     thread). Nothing is thrown across the ABI.
  *   - A plan owns its workspace (dust, Gram partials, Cholesky factors, solve buffers, grid-barrier counters). Calls on
  *     one plan must not overlap in time (same stream, or externally ordered); use one plan per concurrent stream.
+ *   - Calls on several streams share the device's compute units (CUs). The Cholesky's flag waits need all workgroups of
+ *     a factorisation resident, one per CU, beside the other streams' workgroups that wait in turn. A factorisation
+ *     that prefers one XCD runs spread over all eight when another stream is in the way, so what a call needs of each
+ *     XCD's 32 CUs is ceil(SPANQR_Q_CHOL_GRID / 8) for every matrix of its launch, and its solve's workgroups come on
+ *     top, ceil(K / SPANQR_Q_SOLVE_ROWS) / 8 where SPANQR_Q_SOLVE_ROWS > 0. Any number of streams is safe while one
+ *     call's first number and the others' sums stay within 32: two streams of any single-matrix calls, three of
+ *     768 x 512. A wait that gives up all the same shows as NaN and in spanqr_plan_status.
  */
 #ifndef SPANQR_H
 #define SPANQR_H
@@ -248,6 +255,18 @@ int spanqr_chol32(spanqr_plan* plan, const float* G, long ldg, const float* tau,
  * comes out NaN. Applies to launches made after the call (a captured graph keeps the value it was captured with).
  * Not thread-safe with concurrent launches; restore the default (1048576) afterwards. */
 int spanqr_debug_spin_limit(unsigned polls);
+
+/* Testing only (no counterpart in the reference): how long, in ticks of the 100 MHz wall clock, a factorisation that
+ * prefers one XCD waits for all its workgroups to be there before it runs spread over the device (default 1000). With 0
+ * every such factorisation runs spread; the results are the same bits. Applies to launches made after the call (a captured
+ * graph keeps its value). Not thread-safe with concurrent launches; restore the default afterwards. */
+int spanqr_debug_place_ticks(unsigned ticks);
+
+/* Testing only (no GPU needed): what the workgroup at launch index idx of a Cholesky launch does, for `grid` workgroups
+ * per factorisation and nz matrices, m = 8 (each matrix preferably on one XCD, matrix 0 on XCD `slot`) or 1 (spread,
+ * slot 0): out3 = {the Cholesky's workgroup or -1, its matrix (or, with -1, the rank among the solve's workgroups), 1 if
+ * of the set that runs on one XCD}. */
+int spanqr_debug_chol_role(int idx, int grid, int nz, int m, int slot, int* out3);
 
 /* ---- fp64 clamped Cholesky (kchol.chol64, candidates/kchol.py:47-57 -> chol_f64, candidates/cuk/chol.cu:278-281) ----
  * A plan holds the flag words of one n x n factorisation (n a multiple of 32 up to 1024); one plan per concurrent

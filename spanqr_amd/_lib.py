@@ -54,6 +54,8 @@ SIGNATURES = {
     "spanqr_plan_status": (_I, [_P, _P]),
     "spanqr_chol32": (_I, [_P, _P, _L, _P, _P, _L, _P, _P]),
     "spanqr_debug_spin_limit": (_I, [ctypes.c_uint]),
+    "spanqr_debug_place_ticks": (_I, [ctypes.c_uint]),
+    "spanqr_debug_chol_role": (_I, [_I, _I, _I, _I, _I, _P]),
     "spanqr_chol64_plan_create": (_I, [_I, _I, ctypes.POINTER(ctypes.c_void_p)]),
     "spanqr_chol64_plan_destroy": (None, [_P]),
     "spanqr_chol64": (_I, [_P, _P, _L, _P, _P, _P, _P, _P, _P]),

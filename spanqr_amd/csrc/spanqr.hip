@@ -57,8 +57,11 @@ constexpr int BAR_STRIDE = 64;
 constexpr int KCH_MAX_R = 1024;    // kcholf at full width: r a multiple of 32 up to this
 constexpr int CH_MAXROW = KCH_MAX_R / CB;   // tiles in a tile row at most
 // Cholesky flags: [nb * nb] panel flags, [nb] hand-over flags, then a call counter per Cholesky workgroup (99 at
-// r = 1024, checked below)
+// r = 1024, checked below) -- with the one-XCD placement two counters (the one-XCD and the spread workgroups) and an
+// arrival word -- and, in the last 128-byte line, the call's place
 constexpr int FLAG_STRIDE = 1280;
+constexpr int PLACE_WORD = FLAG_STRIDE - 32;
+static_assert(FLAG_STRIDE % 32 == 0, "the place word's line holds nothing else");
 constexpr int CC_STRIDE = 16;      // uint32 words between the solve's column counters (one 64-byte line each)
 
 // The caller's matrices of one launch, passed by value (a captured graph keeps the pointers): matrix z of the
@@ -1124,6 +1127,64 @@ __device__ __forceinline__ uint32_t xcc_id() {
     return __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11));   // HW_REG_XCC_ID, 4 bits
 }
 
+// Where a factorisation that may run on one XCD runs is settled on the device, once per call: *place becomes 2 ep + 1
+// (one XCD) or 2 ep (spread) for call number ep, by compare-and-swap, and the first decision stands (chol_body).
+__device__ __forceinline__ bool place_known(uint32_t v, uint32_t ep) { return (v >> 1) == (ep & 0x7fffffffu); }
+// v: what the caller last read there
+__device__ __forceinline__ bool decide_place(uint32_t* place, uint32_t v, uint32_t ep, bool one_xcd) {
+    while (!place_known(v, ep)) {
+        const uint32_t want = 2 * ep + (one_xcd ? 1u : 0u);
+        if (__hip_atomic_compare_exchange_strong(place, &v, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+            return one_xcd;
+    }
+    return (v & 1u) != 0u;
+}
+// Wait for the decision (a workgroup of the spread set, or with `first` an owner part on one XCD, which as a rule learns
+// it by seeing the call's first flag), and after `ticks` of the wall clock settle for spread: so this wait always
+// ends, whatever else is resident. Called by one lane.
+__device__ __forceinline__ bool wait_place(uint32_t* place, uint32_t ep, uint32_t ticks, const uint32_t* first = nullptr) {
+    const uint64_t t0 = stamp_clock();
+    for (;;) {
+        if (first != nullptr) {
+            for (int n = 0; n < 16; ++n) {
+                if (__hip_atomic_load(first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ep) return true;
+                __builtin_amdgcn_s_sleep(1);
+            }
+        } else {
+            __builtin_amdgcn_s_sleep(16);
+        }
+        const uint32_t v = __hip_atomic_load(place, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (place_known(v, ep)) return (v & 1u) != 0u;
+        if (stamp_clock() - t0 >= ticks) return decide_place(place, v, ep, false);
+    }
+}
+// The one-XCD set's workgroup 0, one wavefront: take the place once all other workgroups of the set have posted (arr) that
+// they are on this XCD. v: what *place held before the call
+__device__ __forceinline__ bool take_place(uint32_t* place, uint32_t v, const uint32_t* arr, int grid, uint32_t ep,
+                                           uint32_t ticks) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t t0 = stamp_clock();
+    bool here = ticks != 0;
+    for (int b0 = 1; b0 < grid && here; b0 += 64) {
+        const int q = b0 + lane;
+        uint32_t a = 0;
+        for (;;) {
+            a = q < grid ? __hip_atomic_load(arr + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+            if (__all(q >= grid || (a >> 4) == (ep & 0x0fffffffu))) break;
+            if (stamp_clock() - t0 >= ticks) {
+                here = false;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        here = here && __all(q >= grid || (a & 15u) == xcc_id());
+    }
+    bool one = false;
+    if (lane == 0) one = decide_place(place, v, ep, here);
+    return one;   // (lane 0's)
+}
+
 // Barrier of some waves of a workgroup while the others keep running: an LDS counter that each participating
 // wave's lane 0 bumps after its own LDS writes have completed, then waits for (bounded) until it reaches `target`
 // (the number of participants times the number of times this barrier has been passed).
@@ -1405,27 +1466,35 @@ size_t chol_lds_bytes(int r, int w) {
 // the two CUs are: measured as a round trip of two workgroups with 8 KB each way, 2.8 us (3.7 with other workgroups
 // writing) across XCDs, where the producer must write its L2 back and the consumer invalidate its own, and 1.26 us
 // within one XCD, where the L2 is the common memory: the stores' completion, a flag in the L2, and loads that pass by
-// the L1. So the launch places the workgroups of a factorisation on one XCD when they fit there (launch index
-// congruent mod 8), and they check where they are: each owner part posts its XCD at its start, workgroup 0 compares
-// them during step 0 and says which protocol the call takes in bit 0 of every flag (the first flag an owner waits
-// for, (0, 0), is stored for all XCDs to see). What the solve reads from other XCDs, the packed operands, is then
-// written through the L2 when it is stored, so no L2 write-back is left in the kernel. XCD false: a launch that is
-// spread from the start (r > 608, where the workgroups do not fit on one XCD, and r <= 160, where there is next to
-// nothing to hand over) runs without any of this: the check, the loads past the L1 and the second form of every store
-// cost it 0.4 us per launch (r <= 160) and 2 us (3001 x 736).
-static_assert(2 * chol_workgroups(CH_MAXROW, OWNER_W) <= FLAG_STRIDE - CH_MAXROW * (CH_MAXROW + 1),
-              "a call counter and an arrival word per Cholesky workgroup after the panel and hand-over flags");
+// the L1. So where the workgroups of a factorisation fit on one XCD the launch puts them there (launch index congruent
+// mod 8). What the solve reads from other XCDs, the packed operands, is written through the L2 when it is stored, so
+// no L2 write-back is left in the kernel.
+// The XCD may not have the room: another stream's factorisation may be there, of this process or another. The flag
+// waits need every workgroup resident, and two factorisations that each hold a part of one XCD would starve each
+// other. So the launch holds the factorisation's workgroups twice, on one XCD and spread over all of them, and one of
+// the two sets runs: every one-XCD owner part posts that it is here and on which XCD, workgroup 0 takes the place when
+// all are (during step 0: the tile factor hides the wait), and where that has not happened after `ticks`, any workgroup
+// of either set, whichever looks first, settles for spread. Until the decision no workgroup of either set stores
+// anything but the values the other would, the set that lost leaves at once, and a one-XCD set that won is resident
+// as a whole and waits for nothing outside it. The spread set needs what it would need alone: a few CUs on each XCD.
+// XCD false: a launch that is only spread (r > 608, where the workgroups do not fit on one XCD, and r <= 160, where
+// there is next to nothing to hand over) runs without any of this: the check, the loads past the L1 and the second
+// form of every store cost it 0.4 us per launch (r <= 160) and 2 us (3001 x 736).
+static_assert(CH_MAXROW * (CH_MAXROW + 1) + chol_workgroups(CH_MAXROW, OWNER_W) <= PLACE_WORD,
+              "a call counter per Cholesky workgroup after the panel and hand-over flags");
 
 __device__ __forceinline__ void credit(uint32_t* colcnt, int k) {
     if (colcnt != nullptr) __hip_atomic_fetch_add(colcnt + (size_t)k * CC_STRIDE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The Cholesky of workgroup b of matrix z (the pointers address matrix 0 of the launch).
+// The Cholesky of workgroup b of matrix z (the pointers address matrix 0 of the launch); local (XCD only): of the set on
+// one XCD.
 template <bool STAMP, bool XCD>
 __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A, int r, const double* __restrict__ npart,
                                           int nnp, float alpha, float tau_rel, float* L, float* Li, float* Lp,
                                           uint32_t* bar, uint32_t* flags, float* scal, uint64_t* stamps, uint32_t lim,
-                                          uint32_t* colcnt, int ow, int ngrid, const float* tau_ptr = nullptr) {
+                                          uint32_t* colcnt, int ow, int ngrid, const bool local, uint32_t ticks,
+                                          const float* tau_ptr = nullptr) {
     extern __shared__ float4 chol_lds[];
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int nb = r / CB;
@@ -1443,16 +1512,28 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
     uint32_t* err = bar + 2;
     uint32_t* flagL = flags;
     uint32_t* flagT = flags + nb * nb;
-    uint32_t* cnt = flags + nb * nb + nb;
-    uint32_t* arr = cnt + ngrid;           // arrival words: (call number, XCD) of each owner part
+    uint32_t* cnt = flags + nb * nb + nb + (XCD && !local ? ngrid : 0);
+    uint32_t* arr = flags + nb * nb + nb + 2 * ngrid;   // arrival words: (call number, XCD) of each one-XCD owner part
+    uint32_t* place = flags + PLACE_WORD;
     bool dead = false;
-    if (STAMP && b == 0 && tid == 0) stamps[0] = stamp_clock();
     const uint32_t calls = cnt[b];         // (read first, used only once the first tiles are here)
-    // misc: [0..2] nrm, shift, tau, [3] local; workgroup 0's LDS words: [4] the row wavefronts' barrier counter, [5] the last step
+    const uint32_t place0 =
+        XCD && local ? __hip_atomic_load(place, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    // misc: [0..2] nrm, shift, tau, [3] the call's place is this XCD, [16] the same for the spread set; workgroup 0's LDS words: [4] the row wavefronts' barrier counter, [5] the last step
     // whose L(j+2, j) is formed, [6] the halves of L(j+2, j-1) formed, [7] the tile factor's pairs done; [32..63] the tile factor's diagonal (piv q),
     // [64..127] its per-pair scalars
     float* misc = reinterpret_cast<float*>(chol_lds);
     Tile* tiles = reinterpret_cast<Tile*>(misc + 256);
+    if (XCD && !local) {
+        uint32_t* gone = reinterpret_cast<uint32_t*>(misc + 16);
+        if (tid == 0) *gone = wait_place(place, calls + 1, ticks) ? 1u : 0u;
+        __syncthreads();
+        if (*gone) {
+            if (tid == 0) cnt[b] = calls + 1;
+            return;
+        }
+    }
+    if (STAMP && b == 0 && tid == 0) stamps[0] = stamp_clock();
     // an owner part: tile row oi, tiles T(oi, os..oe-1)
     int oi = 0, os = 0, oe = 0;
     if (b > 0) owner_part(b, nb, ow, oi, os, oe);
@@ -1469,6 +1550,8 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                                      [&](int q) { return A + (size_t)CB * oi * r + (size_t)CB * (os + q); });
         }
     }
+    // (posted here, beside the first loads: workgroup 0's tile factor then hides its wait for it)
+    if (XCD && local && b > 0 && w == 3 && lane == 0) set_flag(arr + b, ((calls + 1) << 4) | xcc_id());
     if (w == 0) {
         // lane sums in index order, the partials loaded eight at a time (one memory latency per eight)
         double s = 0.0;
@@ -1510,9 +1593,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
         }
     }
     __syncthreads();
-    const uint32_t ep = calls + 1;         // this call's number (every workgroup runs every call)
-    bool local = false;                    // this call's protocol (see above), known after workgroup 0's first flag
-    uint32_t fv = XCD ? 0u : 2 * ep;       // then the call's flag value: 2 ep + local
+    const uint32_t ep = calls + 1;         // this call's number (every workgroup of both sets counts every call)
     float* pq = misc + 32;
 
     if (b == 0) {
@@ -1539,8 +1620,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
             const size_t o = (size_t)CB * j;
             if (lane == 0) {
                 release_to(local);
-                if (j == 0) set_flag(flagL, fv);   // (for every XCD: the owners do not know the protocol yet)
-                else set_flag_to(flagL + j * nb + j, fv, local);
+                set_flag_to(flagL + j * nb + j, ep, local);
                 // the release covers column j-1's operands (stored in step j); column nb-2 is credited in the last
                 // step, column nb-1 by wave 0
                 if (j >= 1 && j < nb - 1) credit(colcnt, j - 1);
@@ -1554,26 +1634,6 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 store_tile_op<XCD>(Lp + (size_t)op_pair(j + 2, j) * CB * CB, z.P2[q], lane, 64);
             }
         };
-        // wave 3, step 0: the XCD of every owner part, once all have posted theirs
-        auto find_protocol = [&]() {
-            bool same = true;
-            for (int b0 = 1; b0 < ngrid; b0 += 64) {
-                const int q = b0 + lane;
-                uint32_t v = 0, polls = 0;
-                while (!dead) {
-                    v = q < ngrid ? __hip_atomic_load(arr + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-                    const bool ok = q >= ngrid || (v >> 4) == (ep & 0x0fffffffu);
-                    if (__all(ok)) break;
-                    if (++polls > lim) {
-                        if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        dead = true;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-                same = same && __all(q >= ngrid || (v & 15u) == xcc_id());
-            }
-            if (lane == 0) reinterpret_cast<uint32_t*>(misc)[3] = (same && !dead) ? 1u : 0u;
-        };
         // Waves 0 and 7 take turns: at step j one factors T(j, j) (wave 0 at even j), the other forms tile row j+1's
         // look-ahead beside it and so ends the step holding T(j+1, j+1) through block j -- the next step's tile, in
         // the registers of the wavefront that factors it.
@@ -1581,6 +1641,10 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
         uint32_t* fcnt = reinterpret_cast<uint32_t*>(misc + 7);     // the factor's pairs done: 16 j + p + 1
         f32x16 C;                                                   // T(j, j) (factor) or T(j+1, j+1) (look-ahead)
         if (w == 0) load_sym(C, z.D[0]);
+        if (XCD && local && w == 3) {
+            const bool one = take_place(place, place0, arr, ngrid, ep, ticks);
+            if (lane == 0) reinterpret_cast<uint32_t*>(misc)[3] = one ? 1u : 0u;
+        }
         for (int j = 0; j < nb; ++j) {
             const int p = j & 1, pp = p ^ 1;
             const int wf = p ? 7 : 0, wr = 7 - wf;                  // this step's factor and look-ahead wavefronts
@@ -1616,7 +1680,6 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
             } else if (w == 3) {
                 // wave 3 publishes the previous step
                 if (j >= 1) publish(j - 1);
-                else if (XCD) find_protocol();
                 if (colcnt != nullptr && j == nb - 1 && nb >= 2) {   // column nb-2's operands, stored just now
                     release_to(local);
                     if (lane == 0) credit(colcnt, nb - 2);
@@ -1638,7 +1701,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                     load_tiles<4, 256>(&R2[t0], 4 - t0, r, 1u << (3 - t0), shift, wl,
                                        [&](int q) { return rowp + CB * (j - 1 + t0 + q); });
                 } else {
-                    if (lane == 0) wait_flag(flagT + i2, fv, err, dead, lim, local);
+                    if (lane == 0) wait_flag(flagT + i2, ep, err, dead, lim, local);
                     if (STAMP && w == 1 && lane == 0) stamps[2 + 6 * nb + j] = stamp_clock();
                     __builtin_amdgcn_wave_barrier();
                     // each wavefront fetches the parts of row j+2 that it alone reads and updates below: waves 1 and
@@ -1728,19 +1791,15 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 if (STAMP && w == 1 && lane == 0) stamps[2 + 4 * nb + j] = stamp_clock();
             }
             __syncthreads();
-            if (XCD && j == 0) {
-                local = reinterpret_cast<uint32_t*>(misc)[3] != 0u;
-                fv = 2 * ep + (local ? 1u : 0u);
-            }
+            if (XCD && local && j == 0 && reinterpret_cast<uint32_t*>(misc)[3] == 0u) break;
             // start the L2 write-back of this step's stores now; the publication at the next step's start then
             // finds the lines clean
             if (w == 4 && !local) asm volatile("buffer_wbl2 sc1" ::: "memory");
             if (STAMP && tid == 0) stamps[2 + 4 * j] = stamp_clock();
         }
-        if (w == 3) publish(nb - 1);
+        if (w == 3 && !(XCD && local && reinterpret_cast<uint32_t*>(misc)[3] == 0u)) publish(nb - 1);
         if (STAMP && tid == 0) stamps[1 + 4 * nb] = stamp_clock();
     } else {
-        if (XCD && tid == 0) set_flag(arr + b, (ep << 4) | xcc_id());
         // Owner part: tile row i, tiles T(i, s..e-1) in LDS. rt[k - s] = T(i, k); pn[k - s] = L(k, j) of the current
         // column block for the part's columns k < i; li = Li_j; pin = L(i, j) when another part of the row holds
         // T(i, j). Each part runs blocks j until its tiles are done: the last part (which holds T(i, i)) to block
@@ -1760,7 +1819,14 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
         Tile& pin = tiles[2 * pw + 1];
         const int l16 = lane & 15, lk = lane >> 4, qd = w & 3, bi = qd >> 1, bj = qd & 1;
         const bool upq = (bi == 0 && bj == 1);
-        for (int j = 0; j <= jl; ++j) {
+        int j0 = 0;
+        if (XCD && local) {
+            // whether the call runs here
+            if (tid == 0) reinterpret_cast<uint32_t*>(misc)[3] = wait_place(place, ep, ticks, flagL) ? 1u : 0u;
+            __syncthreads();
+            if (reinterpret_cast<uint32_t*>(misc)[3] == 0u) j0 = jl + 1;
+        }
+        for (int j = j0; j <= jl; ++j) {
             const bool q4 = w < 4;
             const bool mine = j >= s;                               // this part holds T(i, j): L(i, j) is its output
             const bool hand = last && j + 4 == i;                   // the block after which row i is handed over
@@ -1783,29 +1849,9 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 } else if (lane == nk + 1 && !mine && j >= 1) {
                     f = flagL + i * nb + j;
                 }
-                if (XCD && j == 0) {
-                    // the call's first flag, (0, 0) alone, in either protocol's value
-                    uint32_t polls = 0, got = 0;
-                    while (!dead) {
-                        got = __hip_atomic_load(flagL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        if ((got >> 1) == (ep & 0x7fffffffu)) break;
-                        if (++polls > lim) {
-                            if (lane == 0) __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            dead = true;
-                        }
-                        __builtin_amdgcn_s_sleep(1);
-                    }
-                    if (lane == 0) reinterpret_cast<uint32_t*>(misc)[3] = dead ? 0u : got & 1u;
-                    if (dead || (got & 1u) == 0u) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                } else {
-                    wait_flags_wave(f, fv, err, dead, lim, local);
-                }
+                wait_flags_wave(f, ep, err, dead, lim, local);
             }
             __syncthreads();
-            if (XCD && j == 0) {
-                local = reinterpret_cast<uint32_t*>(misc)[3] != 0u;
-                fv = 2 * ep + (local ? 1u : 0u);
-            }
             if (hst) stamps[2 + 10 * nb + 6 * i] = stamp_clock();
             if (bst) bs[0] = stamp_clock();
             // one batch: Li_j; per column k, the finished L(j+1, j) or T(k, j) through block j-1; T(i, j) into pin
@@ -1908,7 +1954,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 if (hst) stamps[7 + 10 * nb + 6 * i] = stamp_clock();
                 if (tid == 0) {
                     release_to(local);
-                    set_flag_to(flagT + i, fv, local);
+                    set_flag_to(flagT + i, ep, local);
                     if (mine) credit(colcnt, j);   // L(i, i-4)'s packed form
                 }
                 if (hst) stamps[5 + 10 * nb + 6 * i] = stamp_clock();
@@ -1920,7 +1966,7 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
                 if (pub || mine) {
                     release_to(local);
                     if (lane == 0) {
-                        if (pub) set_flag_to(flagL + i * nb + j + 1, fv, local);
+                        if (pub) set_flag_to(flagL + i * nb + j + 1, ep, local);
                         if (mine) credit(colcnt, j);
                     }
                 }
@@ -1932,36 +1978,50 @@ __device__ __forceinline__ void chol_body(const int b, const size_t z, float* A,
     if (tid == 0) cnt[b] = ep;
 }
 
-// The Cholesky workgroup b of matrix z at launch index idx, or -1. Matrices m q .. m q + m - 1 have their `grid`
-// workgroups at the indices m (q grid + b) + k: with m = NXCD the hardware's round robin puts a matrix on one XCD, with
-// m = 1 its workgroups are spread over the XCDs. An index that is no Cholesky workgroup (a gap of a last group of
-// fewer than m matrices, or past them all) gets its rank among such indices in `other`.
+// What the workgroup at launch index idx does; the hardware's round robin runs index i on XCD i mod 8. m = 1: the nz grid
+// workgroups of the factorisations, spread over the XCDs, then the solve's. m = NXCD: matrix z's workgroups on XCD (z +
+// slot) mod 8, matrix after matrix; on every XCD then an eighth of the same workgroups once more, the spread set
+// (chol_body: one of the two sets runs); then the solve's, first where the XCD has fewer factorisations. So on every
+// XCD a factorisation's workgroups have lower indices than the solve's, are dispatched first and never wait on one.
 constexpr int NXCD = 8;
 constexpr int XCD_MIN_R = 160;   // up to two owner parts: spread, 1024 x 160 141.8 us per call, on one XCD 143.7 (192: 153.2, 150.8)
-static_assert(NXCD == 8, "chol_role's shift");
-// (Divisions only where a launch has more than one group of matrices: at the head of every workgroup they cost ~1 us.)
-__device__ __forceinline__ int chol_role(int idx, int grid, int nz, int m, int& z, int& other) {
-    const int sh = m == NXCD ? 3 : 0, s = idx >> sh, k = idx & (m - 1);
-    int q = 0;
-    if (nz > m) {
-        q = s / grid;
-        if (m * q >= nz) {
-            other = idx - nz * grid;
-            return -1;
-        }
-    } else if (s >= grid) {
-        other = idx - nz * grid;
-        return -1;
+static_assert(NXCD == 8, "chol_role's shifts");
+struct CholRole {
+    int b;         // the Cholesky's workgroup, or -1: a solve workgroup or nothing
+    int z;         // its matrix, or the solve's rank
+    bool local;    // of the set on one XCD
+};
+// (Divisions only where a launch has more than one matrix: at the head of every workgroup they cost ~1 us.)
+__host__ __device__ inline CholRole chol_role(int idx, int grid, int nz, int m, int slot) {
+    const int nwg = nz * grid;
+    if (m == 1) {
+        if (idx >= nwg) return {-1, idx - nwg, false};
+        const int z = nz == 1 ? 0 : idx / grid;
+        return {idx - z * grid, z, false};
     }
-    z = m * q + k;
-    if (z < nz) return s - q * grid;
-    const int nlast = nz - m * q;
-    other = (s - q * grid) * (m - nlast) + k - nlast;
-    return -1;
+    // row s of XCD k (counted from slot): X rows of whole factorisations, E of the spread set, then the solve's. The
+    // first nl XCDs have one factorisation more than the others.
+    const int s = idx >> 3, k = (idx - slot) & 7, groups = (nz + 7) >> 3, nl = nz - 8 * (groups - 1);
+    const int mine = k < nl ? groups : groups - 1, X = mine * grid, E = (nwg + 7) >> 3;
+    if (s < X) {
+        const int q = groups == 1 ? 0 : s / grid;
+        return {s - q * grid, 8 * q + k, true};
+    }
+    if (s < X + E) {
+        const int u = 8 * (s - X) + k;
+        const int z = nz == 1 ? 0 : u / grid;
+        if (u < nwg) return {u - z * grid, z, false};
+        return {-1, 1 << 30, false};   // (past the set: nothing)
+    }
+    const int hi = groups * grid + E;   // from this row on every XCD runs the solve
+    if (s >= hi) return {-1, (8 - nl) * grid + 8 * (s - hi) + k, false};
+    return {-1, (8 - nl) * (s - X - E) + k - nl, false};
 }
-// launch indices of the Cholesky's workgroups with `others` further ones
-int chol_launch_size(int grid, int nz, int m, int others) {
-    return std::max((nz + m - 1) / m * m * grid, nz * grid + others);
+// launch indices of the Cholesky's workgroups with `solves` of the solve
+int chol_launch_size(int grid, int nz, int m, int solves) {
+    if (m == 1) return nz * grid + solves;
+    const int groups = (nz + 7) / 8, nl = nz - 8 * (groups - 1);
+    return 8 * (groups * grid + (nz * grid + 7) / 8 + std::max(0, (solves - (8 - nl) * grid + 7) / 8));
 }
 
 // tau_ptr (nnp == 0 only; may be null): the absolute pivot floor read from device memory instead of tau_rel (chol32
@@ -1970,12 +2030,12 @@ template <bool STAMP, bool XCD>
 __global__ __launch_bounds__(512) void k_chol(float* A, int r, const double* __restrict__ npart, int nnp, float alpha,
                                               float tau_rel, float* L, float* Li, float* Lp, uint32_t* bar,
                                               uint32_t* flags, float* scal, uint64_t* stamps, uint32_t lim, int ow,
-                                              int grid, int nz, int m, const float* tau_ptr) {
-    int z = 0, other = 0;
-    const int b = chol_role(blockIdx.x, grid, nz, m, z, other);
-    if (b < 0) return;
-    chol_body<STAMP, XCD>(b, z, A, r, npart, nnp, alpha, tau_rel, L, Li, Lp, bar, flags, scal, stamps, lim, nullptr, ow, grid,
-                     tau_ptr);
+                                              int grid, int nz, int m, int slot, uint32_t ticks,
+                                              const float* tau_ptr) {
+    const CholRole role = chol_role(blockIdx.x, grid, nz, m, slot);
+    if (role.b < 0) return;
+    chol_body<STAMP, XCD>(role.b, role.z, A, r, npart, nnp, alpha, tau_rel, L, Li, Lp, bar, flags, scal, stamps, lim,
+                          nullptr, ow, grid, role.local, ticks, tau_ptr);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -2364,13 +2424,12 @@ __device__ __forceinline__ void trsm_wave_body(const int g, const int z, const M
     }
 }
 
-// One pass's Cholesky and its solve in one launch: workgroups [0, nz grid) run the Cholesky of matrix
-// b / grid (workgroup b % grid), the rest the solve of matrix b' / nrb (row blocks of 16 RB rows, b' % nrb), the
-// solve following the factor column by column through the counters (the Cholesky's workgroups come first, so they
-// are dispatched first and never wait on a solve workgroup). Pointers address matrix 0 of the launch.
+// One pass's Cholesky and its solve in one launch (chol_role): solve workgroup u takes row blocks (16 RB rows) u % nrb
+// of matrix u / nrb and follows the factor column by column through the counters. Pointers address matrix 0 of the
+// launch.
 struct CholArgs {
     float* A; const double* npart; float* L; float* Li; float* Lp; uint32_t* bar; uint32_t* flags; float* scal;
-    uint32_t* colcnt; float alpha, tau_rel; int r, nnp, nz, grid, m, ow; uint32_t lim;   // m: chol_role; ow: owner part width
+    uint32_t* colcnt; float alpha, tau_rel; int r, nnp, nz, grid, m, slot, ow; uint32_t lim, ticks;   // m, slot: chol_role; ow: owner part width
 };
 struct SolveArgs {
     MatsIn A; MatsOut Y; const uint32_t* amax_part; const float* Z; float* scal; long lda, ldz, ldy; float eps;
@@ -2381,13 +2440,13 @@ struct SolveArgs {
 // with NBC = RB column blocks (eight row blocks per workgroup).
 template <bool PASS1, int Q, int RB, bool XCD>
 __global__ __launch_bounds__(64 * TRSM_NW) void k_chol_solve(const CholArgs c, const SolveArgs t) {
-    int z = 0, b = 0;
-    const int cb = chol_role(blockIdx.x, c.grid, c.nz, c.m, z, b);
-    if (cb >= 0) {
-        chol_body<false, XCD>(cb, z, c.A, c.r, c.npart, c.nnp, c.alpha, c.tau_rel, c.L, c.Li, c.Lp, c.bar, c.flags, c.scal,
-                         nullptr, c.lim, c.colcnt, c.ow, c.grid);
+    const CholRole role = chol_role(blockIdx.x, c.grid, c.nz, c.m, c.slot);
+    if (role.b >= 0) {
+        chol_body<false, XCD>(role.b, role.z, c.A, c.r, c.npart, c.nnp, c.alpha, c.tau_rel, c.L, c.Li, c.Lp, c.bar, c.flags,
+                              c.scal, nullptr, c.lim, c.colcnt, c.ow, c.grid, role.local, c.ticks);
         return;
     }
+    const int b = role.z;
     if (b >= c.nz * t.nrb) return;   // a gap that holds no solve workgroup
     const int zs = c.nz == 1 ? 0 : b / t.nrb, rb = b - zs * t.nrb;
     if constexpr (Q == 0)
@@ -2876,6 +2935,16 @@ thread_local std::string g_err;
 // polls of one bounded wait before the Cholesky gives up on it (spanqr_debug_spin_limit lowers it for the tests of
 // the failure path)
 uint32_t g_spin_limit = SPIN_LIMIT;
+// Ticks of the 100 MHz wall clock after which a factorisation that is not yet whole on one XCD runs spread
+// (spanqr_debug_place_ticks). On an idle device its workgroups are there within 3 us (2.5 us is too short: 768 x 512 312.8
+// us per call instead of 290); where another stream holds the XCD it is the price of trying. Two streams of calls side
+// by side, us per pair of calls with 5 / 10 / 20 us: 768 x 512 334 / 339 / 331..384, 2048 x 512 496 / 512 / 535 (spread
+// only, before the one-XCD form: 339 and 461).
+constexpr uint32_t PLACE_TICKS = 1000;
+uint32_t g_place_ticks = PLACE_TICKS;
+// the XCD of a plan's first matrix: plans take turns, so that factorisations of two streams mostly want different ones
+std::atomic<uint32_t> g_next_slot{0};
+int next_slot() { return (int)(g_next_slot.fetch_add(1, std::memory_order_relaxed) % NXCD); }
 
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 int fail(int code, const char* fmt, ...) {
@@ -2924,6 +2993,7 @@ struct spanqr_plan {
     int nnp = 0;              // norm partials per matrix the Gram writes (16 per 64x64 tile, or 1 per 32x32 tile)
     int owner_w = OWNER_W;    // tiles per Cholesky owner part at most
     int chol_m = 1;           // NXCD: each matrix's Cholesky workgroups on one XCD; 1: spread (chol_role)
+    int chol_slot = 0;        // with NXCD: the XCD of matrix 0
     bool trsm_rows = false;   // solve with a wavefront pair per 16 rows (k_trsm_rows) instead of k_trsm
     int solve_rb = 0;         // row blocks per solve workgroup in the Cholesky's launch (0: separate launches)
     int solve_nrb = 0;        // solve workgroups per matrix there
@@ -3107,7 +3177,7 @@ int launch_chol(spanqr_plan* p, float alpha, float tau, float* scal, hipStream_t
         auto* kernel = stamp ? (xcd ? k_chol<true, true> : k_chol<true, false>)
                              : (xcd ? k_chol<false, true> : k_chol<false, false>);
         kernel<<<grid, 512, lds, st>>>(A, p->r, np, nnp, alpha, tau, L, Li, Lp, bar, flags, sc, p->stamps, g_spin_limit,
-                                       p->owner_w, p->chol_grid, nz, p->chol_m, tau_ptr);
+                                       p->owner_w, p->chol_grid, nz, p->chol_m, p->chol_slot, g_place_ticks, tau_ptr);
         HIPCHK(hipGetLastError());
     }
     return SPANQR_OK;
@@ -3315,6 +3385,8 @@ int launch_chol_solve(spanqr_plan* p, float alpha, float tau, float* scal, hipSt
         c.nz = nz;
         c.grid = p->chol_grid;
         c.m = p->chol_m;
+        c.slot = p->chol_slot;
+        c.ticks = g_place_ticks;
         c.ow = p->owner_w;
         c.lim = g_spin_limit;
         SolveArgs t{};
@@ -3536,6 +3608,8 @@ int plan_device_setup(spanqr_plan* p, int device) {
                 int bmax;
                 if (pass == 0) {
                     if (r <= XCD_MIN_R || grid > xcd || (p->batch == 1 && w > 8)) continue;
+                    // (the arrival words and both sets' call counters fit before the place word)
+                    if ((r / CB) * (r / CB + 1) + 3 * grid > PLACE_WORD) continue;
                     bmax = NXCD * std::max(1, xcd * 7 / 8 / grid);
                 } else {
                     if (p->batch == 1 && best_n == 1) break;
@@ -3551,6 +3625,7 @@ int plan_device_setup(spanqr_plan* p, int device) {
                     p->chol_bmax = std::min(bmax, p->batch);
                 }
             }
+        if (p->chol_m == NXCD) p->chol_slot = next_slot();
         if (best_n == 1 << 30)
             return fail(SPANQR_EHIP, "the Cholesky needs %d co-resident workgroups, device holds too few",
                         chol_workgroups(r / CB, OWNER_WMAX));
@@ -4106,6 +4181,21 @@ int spanqr_debug_spin_limit(unsigned polls) {
     return SPANQR_OK;
 }
 
+int spanqr_debug_place_ticks(unsigned ticks) {
+    g_place_ticks = ticks;
+    return SPANQR_OK;
+}
+
+int spanqr_debug_chol_role(int idx, int grid, int nz, int m, int slot, int* out3) {
+    if (idx < 0 || grid < 1 || nz < 1 || (m != 1 && m != NXCD) || slot < 0 || slot >= m || !out3)
+        return fail(SPANQR_EINVAL, "bad arguments");
+    const CholRole role = chol_role(idx, grid, nz, m, slot);
+    out3[0] = role.b;
+    out3[1] = role.z;
+    out3[2] = role.local ? 1 : 0;
+    return SPANQR_OK;
+}
+
 int spanqr_plan_copy_dust(spanqr_plan* p, float* Z, void* stream) {
     if (!p || !Z) return fail(SPANQR_EINVAL, "null argument");
     if (p->blk) return fail(SPANQR_EINVAL, "not available on a column-blocked plan (r > 512)");
@@ -4353,8 +4443,8 @@ int spanqr_orth_f32_noalloc(int K, int r, const float* X, long ldx, float* Q, lo
 // workgroup 0. All products are v_mfma_f64_16x16x4_f64 chains in ascending k, which round like sequential fmas.
 // What bounds it: the chain of 32-column steps, each a tile factor (a serial chain of 32 pivots) and two products on
 // one CU, and beside it the loop through row j+2's part (Li_j, panel, update, hand-over), so the workgroups of a
-// factorisation sit on one XCD where they fit and hand over through its L2 (n <= 608; the protocol of the fp32
-// factorisation, with the same check of where the workgroups are).
+// factorisation sit on one XCD where they fit and hand over through its L2 (n <= 608; as the fp32 factorisation, with a
+// second, spread set of workgroups for a call that finds no room there).
 // Measured, us per call, before (a workgroup per tile, scalar fma products, hand-overs across XCDs, a launch to clear the
 // flags) and now: n = 32 59.6 / 22.1, 256 476 / 100, 512 957 / 193, 1024 (spread) 1980 / 423; ~12 us per 32 columns, of
 // which the tile factor is ~7.
@@ -4369,7 +4459,7 @@ constexpr int C64_TS = CB + 4;   // row stride in doubles: 16-byte rows, and an 
 typedef double TileD[CB][C64_TS];
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int C64_WG0_TILES = 9;   // D[2], X, P[2], dl[2], li[2]
-constexpr int C64_MISC = 160;      // doubles in front of the tiles: the factor's column broadcasts, the protocol word
+constexpr int C64_MISC = 160;      // doubles in front of the tiles: the factor's column broadcasts, the place
 
 __device__ __forceinline__ f64x4 mfma64(double a, double b, f64x4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -4532,16 +4622,17 @@ size_t chol64_lds_bytes(int n, int w) {
     const int nb = n / CB, part = 2 * std::min(nb, w) + 1;
     return (size_t)std::max(part, C64_WG0_TILES) * sizeof(TileD) + C64_MISC * sizeof(double);
 }
-// flag words: [nb] Li_j, [nb] L(j+1, j), [nb] hand-over of row j, [nb nb] L(i, j), then the error word and, per
-// workgroup, a call counter and an arrival word
-__host__ __device__ constexpr int chol64_err_word(int nb) { return nb * nb + 3 * nb; }
+// flag words: the call's place (in a 128-byte line of its own), [nb] Li_j, [nb] L(j+1, j), [nb] hand-over of row j, [nb
+// nb] L(i, j), then the error word and, per workgroup, the call counters of the two sets and an arrival word
+constexpr int C64_FLAGS = 32;
+__host__ __device__ constexpr int chol64_err_word(int nb) { return C64_FLAGS + nb * nb + 3 * nb; }
 
 // wait_flags_wave with the call number in the error word
-__device__ __forceinline__ void wait64(const uint32_t* mine, uint32_t fv, uint32_t* err, uint32_t ep, bool& dead,
+__device__ __forceinline__ void wait64(const uint32_t* mine, uint32_t* err, uint32_t ep, bool& dead,
                                        uint32_t lim, bool local) {
     uint32_t polls = 0;
     while (!dead) {
-        const bool ok = mine == nullptr || __hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == fv;
+        const bool ok = mine == nullptr || __hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ep;
         if (__all(ok)) break;
         if (++polls > lim) {
             if ((threadIdx.x & 63) == 0) __hip_atomic_store(err, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -4561,20 +4652,33 @@ constexpr int C64_OWMAX = 8;   // widest parts: 17 tiles of LDS
 
 __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, long ldg, int n,
                                                 const double* __restrict__ taup, double* L, double* Li, float* Lf,
-                                                float* Lif, uint32_t* flags, int grid, int m, int ow, uint32_t lim) {
-    int zz = 0, other = 0;
-    const int b = chol_role(blockIdx.x, grid, 1, m, zz, other);
+                                                float* Lif, uint32_t* flags, int grid, int m, int slot, int ow,
+                                                uint32_t lim, uint32_t ticks) {
+    const CholRole role = chol_role(blockIdx.x, grid, 1, m, slot);
+    const int b = role.b;
     if (b < 0) return;
     extern __shared__ double2 c64_lds[];
     double* misc = reinterpret_cast<double*>(c64_lds);
-    uint32_t* proto = reinterpret_cast<uint32_t*>(misc + 128);
+    uint32_t* here = reinterpret_cast<uint32_t*>(misc + 128);   // the call's place is this XCD
     TileD* tl = reinterpret_cast<TileD*>(misc + C64_MISC);
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nb = n / CB;
-    uint32_t *fD = flags, *fP = fD + nb, *fH = fP + nb, *fL = fH + nb, *err = flags + chol64_err_word(nb),
-             *cnt = err + 1, *arr = cnt + grid;
-    const uint32_t ep = cnt[b] + 1;   // this call's number (every workgroup runs every call)
-    uint32_t fv = 0;                  // the call's flag value: 2 ep + local
-    bool dead = false, local = false;
+    uint32_t *place = flags, *fD = flags + C64_FLAGS, *fP = fD + nb, *fH = fP + nb, *fL = fH + nb,
+             *err = flags + chol64_err_word(nb), *cnt = err + 1, *arr = cnt + 2 * grid;
+    const bool two = m == NXCD;                        // a set on one XCD and a spread one (chol_body)
+    const bool local = two ? role.local : grid == 1;   // hand-overs stay on this XCD
+    if (two && !local) cnt += grid;
+    const uint32_t ep = cnt[b] + 1;   // this call's number (every workgroup of both sets counts every call)
+    const uint32_t place0 =
+        two && local ? __hip_atomic_load(place, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    bool dead = false;
+    if (two && !local) {
+        if (tid == 0) *here = wait_place(place, ep, ticks) ? 1u : 0u;
+        __syncthreads();
+        if (*here) {
+            if (tid == 0) cnt[b] = ep;
+            return;
+        }
+    }
     auto Lt = [&](int i, int k) { return L + (size_t)CB * i * n + (size_t)CB * k; };
     auto Lft = [&](int i, int k) { return Lf + (size_t)CB * i * n + (size_t)CB * k; };
     const double2 zero = make_double2(0.0, 0.0);
@@ -4582,6 +4686,7 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
     if (b == 0) {
         TileD *D = tl, &X = tl[2], *P = tl + 3, *dl = tl + 5, *li = tl + 7;
         const double tau = *taup;
+        bool gone = false;   // the spread set runs this call
         put_piece(D[0], tid, load_piece(G, ldg, tid));
         if (nb > 1) {
             put_piece(X, tid, load_piece(G + (size_t)CB * ldg, ldg, tid));
@@ -4610,10 +4715,10 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
             } else if (j > 0) {
                 if (w == 4 && lane == 0) {
                     release_to(local);
-                    set_flag_to(fP + j - 1, fv, local);
+                    set_flag_to(fP + j - 1, ep, local);
                 }
                 if (j + 1 < nb) {
-                    wait64(lane == 0 ? fH + j + 1 : nullptr, fv, err, ep, dead, lim, local);
+                    wait64(lane == 0 ? fH + j + 1 : nullptr, err, ep, dead, lim, local);
                     double2 v[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
@@ -4621,29 +4726,14 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
 #pragma unroll
                     for (int u = 0; u < 4; ++u) put_piece(u < 2 ? X : D[1 - q], t4 + 256 * (u & 1), v[u]);
                 }
-            } else if (w == 7) {
-                // where every part is, once all have posted it
-                bool same = true;
-                for (int b0 = 1; b0 < grid; b0 += 64) {
-                    const int o = b0 + lane;
-                    uint32_t v = 0, polls = 0;
-                    while (!dead) {
-                        v = o < grid ? __hip_atomic_load(arr + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-                        if (__all(o >= grid || (v >> 4) == (ep & 0x0fffffffu))) break;
-                        if (++polls > lim) {
-                            if (lane == 0) __hip_atomic_store(err, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            dead = true;
-                        }
-                        __builtin_amdgcn_s_sleep(1);
-                    }
-                    same = same && __all(o >= grid || (v & 15u) == xcc_id());
-                }
-                if (lane == 0) proto[0] = !dead && same;
+            } else if (w == 7 && two && local) {
+                const bool one = take_place(place, place0, arr, grid, ep, ticks);
+                if (lane == 0) *here = one ? 1u : 0u;
             }
             __syncthreads();
-            if (j == 0) {
-                local = proto[0] != 0u;
-                fv = 2 * ep + (local ? 1u : 0u);
+            if (two && local && j == 0 && *here == 0u) {
+                gone = true;
+                break;
             }
             if (j + 1 == nb) break;
             if (w < 4) {
@@ -4659,19 +4749,19 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
             } else {
                 if (w == 4 && lane == 0) {
                     release_to(local);
-                    if (j == 0) set_flag(fD, fv);   // (for every XCD: the parts do not know the protocol yet)
-                    else set_flag_to(fD + j, fv, local);
+                    set_flag_to(fD + j, ep, local);
                 }
                 for (int e = t4; e < CB * CB / 2; e += 256) store_piece(Lt(j + 1, j), n, e, tile_piece(P[q], e));
                 __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
             }
             __syncthreads();
         }
-        outputs(nb - 1, tid, 512);
-        store_piece(Li + (size_t)(nb - 1) * CB * CB, CB, tid, tile_piece(li[(nb - 1) & 1], tid));
+        if (!gone) {
+            outputs(nb - 1, tid, 512);
+            store_piece(Li + (size_t)(nb - 1) * CB * CB, CB, tid, tile_piece(li[(nb - 1) & 1], tid));
+        }
     } else {
-        if (tid == 0)
-            __hip_atomic_store(arr + b, ((ep & 0x0fffffffu) << 4) | xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (two && local && tid == 0) set_flag(arr + b, (ep << 4) | xcc_id());
         int i, s, e;
         owner_part64(b, nb, ow, i, s, e);
         const bool last = e == i + 1;
@@ -4687,36 +4777,21 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
             for (int u = 0; u < C64_OWMAX; ++u)
                 if (s + u < e) put_piece(rt[u], tid, v[u]);
         }
+        bool gone = false;   // the spread set runs this call
         for (int k = s; k < e && k < i; ++k) {   // the upper triangle's tiles
             store_piece(Lt(k, i), n, tid, zero);
             store_piece_f(Lft(k, i), n, tid, zero);
         }
         for (int j = 0; j <= jl; ++j) {
             const bool mine = j >= s;
-            if (w == 0 && (mine || j == 0)) {
-                if (j == 0) {
-                    // the call's first flag, in either protocol's value
-                    uint32_t polls = 0, got = 0;
-                    while (!dead) {
-                        got = __hip_atomic_load(fD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        if ((got >> 1) == (ep & 0x7fffffffu)) break;
-                        if (++polls > lim) {
-                            if (lane == 0) __hip_atomic_store(err, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            dead = true;
-                        }
-                        __builtin_amdgcn_s_sleep(1);
-                    }
-                    if (lane == 0) proto[0] = dead ? 0u : got & 1u;
-                    if (dead || (got & 1u) == 0u) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                } else {
-                    wait64(lane == 0 ? fD + j : nullptr, fv, err, ep, dead, lim, local);
-                }
+            if (w == 0 && two && local && j == 0 && lane == 0) *here = wait_place(place, ep, ticks, fD) ? 1u : 0u;
+            if (two && local && j == 0) {
+                __syncthreads();
+                gone = *here == 0u;
+                if (gone) break;
             }
+            if (w == 0 && mine) wait64(lane == 0 ? fD + j : nullptr, err, ep, dead, lim, local);
             __syncthreads();
-            if (j == 0) {
-                local = proto[0] != 0u;
-                fv = 2 * ep + (local ? 1u : 0u);
-            }
             TileD& lij = mine ? pn[j - s] : in;   // L(i, j): this part's panel, or the other part's
             if (mine) {
                 put_piece(in, tid, load_piece_agent(Li + (size_t)j * CB * CB, CB, tid));
@@ -4729,7 +4804,7 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
                 __syncthreads();
                 if (tid == 0) {
                     release_to(local);
-                    set_flag_to(fL + i * nb + j, fv, local);
+                    set_flag_to(fL + i * nb + j, ep, local);
                 }
                 store_piece_f(Lft(i, j), n, tid, v);
             }
@@ -4739,7 +4814,7 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
                 const uint32_t* f = nullptr;
                 if (lane < nk) f = k0 + lane == j + 1 ? fP + j : fL + (k0 + lane) * nb + j;
                 else if (lane == nk && !mine) f = fL + i * nb + j;
-                wait64(f, fv, err, ep, dead, lim, local);
+                wait64(f, err, ep, dead, lim, local);
             }
             __syncthreads();
             {
@@ -4761,14 +4836,14 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
             }
             __syncthreads();
         }
-        if (last) {
+        if (last && !gone) {
             store_piece(Lt(i, i - 1), n, tid, tile_piece(rt[i - 1 - s], tid));
             store_piece(Lt(i, i), n, tid, tile_piece(rt[i - s], tid));
             __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
             __syncthreads();
             if (tid == 0) {
                 release_to(local);
-                set_flag_to(fH + i, fv, local);
+                set_flag_to(fH + i, ep, local);
             }
         }
     }
@@ -4780,7 +4855,7 @@ __global__ __launch_bounds__(512) void k_chol64(const double* __restrict__ G, lo
 
 struct spanqr_chol64_plan {
     int n = 0, device = 0, nwords = 0;
-    int grid = 0, m = 1, ow = OWNER_W;    // workgroups, NXCD: all on one XCD, tiles per part
+    int grid = 0, m = 1, slot = 0, ow = OWNER_W;   // workgroups; chol_role's m and slot; tiles per part
     uint32_t* flags = nullptr;            // chol64_err_word's layout
     std::atomic<bool> cleared{false};     // a call outside a capture has cleared the flags (later calls only count up)
 };
@@ -4814,8 +4889,9 @@ int spanqr_chol64_plan_create(int n, int device, spanqr_chol64_plan** out) {
     }
     spanqr_chol64_plan* p = new spanqr_chol64_plan;
     p->n = n; p->device = device;
-    p->grid = grid; p->m = m; p->ow = ow;
-    p->nwords = chol64_err_word(nb) + 1 + 2 * grid;
+    p->grid = grid; p->m = grid == 1 ? 1 : m; p->ow = ow;   // (one workgroup is on one XCD anyway)
+    if (p->m == NXCD) p->slot = next_slot();
+    p->nwords = chol64_err_word(nb) + 1 + 3 * grid;
     if (hipMalloc((void**)&p->flags, (size_t)p->nwords * sizeof(uint32_t)) != hipSuccess) {
         delete p;
         return fail(SPANQR_ENOMEM, "flag allocation failed");
@@ -4852,7 +4928,7 @@ int spanqr_chol64(spanqr_chol64_plan* p, const double* G, long ldg, const double
         if (cap == hipStreamCaptureStatusNone) p->cleared.store(true);
     }
     k_chol64<<<chol_launch_size(p->grid, 1, p->m, 0), 512, chol64_lds_bytes(p->n, p->ow), st>>>(
-        G, ldg, p->n, tau, L, Li, Lf, Lif, p->flags, p->grid, p->m, p->ow, SPIN_LIMIT);
+        G, ldg, p->n, tau, L, Li, Lf, Lif, p->flags, p->grid, p->m, p->slot, p->ow, SPIN_LIMIT, g_place_ticks);
     HIPCHK(hipGetLastError());
     return SPANQR_OK;
 }
