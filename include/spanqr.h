@@ -19,11 +19,12 @@
  *     one plan must not overlap in time (same stream, or externally ordered); use one plan per concurrent stream.
  *   - Calls on several streams share the device's compute units (CUs). The Cholesky's flag waits need all workgroups of
  *     a factorisation resident, one per CU, beside the other streams' workgroups that wait in turn. A factorisation
- *     that prefers one XCD runs spread over all eight when another stream is in the way, so what a call needs of each
- *     XCD's 32 CUs is ceil(SPANQR_Q_CHOL_GRID / 8) for every matrix of its launch, and its solve's workgroups come on
- *     top, ceil(K / SPANQR_Q_SOLVE_ROWS) / 8 where SPANQR_Q_SOLVE_ROWS > 0. Any number of streams is safe while one
- *     call's first number and the others' sums stay within 32: two streams of any single-matrix calls, three of
- *     768 x 512. A wait that gives up all the same shows as NaN and in spanqr_plan_status.
+ *     that prefers one XCD runs spread over all eight when another stream is in the way, so of each XCD's 32 CUs a call
+ *     needs about c = SPANQR_Q_CHOL_GRID / 8 per matrix of its launch, and its solve's workgroups may hold s = K / (7
+ *     SPANQR_Q_SOLVE_ROWS) more (0 where that query is 0). Two streams are safe where one call's c and the other's c +
+ *     s are within 32, in one of the two orders: any two of 768 x 512, 2048 x 512, 17408 x 256 and their like, but not
+ *     two of 2048 x 1024 (c = 13, s = 16), which the caller has to order; more streams where that holds of each call
+ *     and all the others together. A wait that gives up all the same shows as NaN and in spanqr_plan_status.
  */
 #ifndef SPANQR_H
 #define SPANQR_H
@@ -61,7 +62,7 @@ enum {
     SPANQR_Q_WORKSPACE_MB = 5,   /* workspace size, MiB (rounded up) */
     SPANQR_Q_DEVICE = 6,
     SPANQR_Q_BATCH = 7,          /* matrices per call the plan holds workspace for */
-    SPANQR_Q_CHOL_BATCH = 8,     /* matrices per Cholesky launch (all their workgroups fit on the device at once) */
+    SPANQR_Q_CHOL_BATCH = 8,     /* matrices per Cholesky launch (their workgroups take at most 7/8 of the device) */
     SPANQR_Q_BLOCKS = 9,         /* column blocks of a column-blocked plan (r > 512, or spanqr_plan_create_borth); 0
                                     otherwise */
     SPANQR_Q_SOLVE_ROWS = 10,    /* rows per solve workgroup when the solve runs in the Cholesky's launch; 0 when

@@ -3595,8 +3595,9 @@ int plan_device_setup(spanqr_plan* p, int device) {
     // goes there (m = NXCD); otherwise its workgroups are spread (m = 1). One matrix takes the narrowest parts, in tiles, that fit on
     // one XCD with at most 8 tiles (12-tile parts there: 671 us per call at 3001 x 736, 6-tile parts spread: 656), or
     // else OWNER_W; a batch the narrowest parts that run its Cholesky in the fewest launches. Each launch
-    // needs all its workgroups resident at once: several matrices take at most 7/8 of an XCD or three quarters of the
-    // device (the margin leaves room for work of other streams).
+    // needs all its workgroups resident at once: several matrices take at most 7/8 of the device where each has an XCD
+    // (28 CUs of each: a spread factorisation of another stream, four workgroups per XCD at r = 512, still fits beside
+    // them) or three quarters of it spread (the margin leaves room for work of other streams).
     {
         const int widths[] = {OWNER_W, 8, 12, OWNER_WMAX};
         int best_n = 1 << 30;
@@ -3610,7 +3611,7 @@ int plan_device_setup(spanqr_plan* p, int device) {
                     if (r <= XCD_MIN_R || grid > xcd || (p->batch == 1 && w > 8)) continue;
                     // (the arrival words and both sets' call counters fit before the place word)
                     if ((r / CB) * (r / CB + 1) + 3 * grid > PLACE_WORD) continue;
-                    bmax = NXCD * std::max(1, xcd * 7 / 8 / grid);
+                    bmax = std::max(1, std::min(NXCD * std::max(1, xcd * 7 / 8 / grid), o * cus * 7 / 8 / grid));
                 } else {
                     if (p->batch == 1 && best_n == 1) break;
                     if (o * cus < grid || (p->batch == 1 && w != OWNER_W)) continue;

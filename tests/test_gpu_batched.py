@@ -8,7 +8,7 @@ import torch
 
 import oracle
 from spanqr_amd import _lib, kcholqr_f, kcholqr_f_many, orth, orth_many
-from spanqr_amd.plan import get_plan, stream_handle
+from spanqr_amd.plan import Plan, get_plan, stream_handle
 from spanqr_amd.qrbench import gen
 
 from checks import assert_bits, gate
@@ -169,3 +169,15 @@ def test_batched_long_splits(cuda):
     for i in range(n):
         assert_bits(Qs[i], kcholqr_f(Xs[i].to(cuda)), f"batch element {i} vs single call")
     assert_bits(Qs[1], oracle.orth(Xs[1].numpy(), plan.split_rows), "element 1 vs oracle")
+
+
+@pytest.mark.parametrize("r", [192, 256, 512, 544, 608, 640, 736, 800, 1024])
+def test_batched_launches_leave_room(cuda, r):
+    """several matrices of one Cholesky launch take at most 7/8 of the compute units, so that a factorisation of another
+    stream finds room on every XCD"""
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    for batch in (2, 8, 13, 32):
+        plan = Plan(r, r, cuda.index, batch)
+        assert 1 <= plan.chol_batch <= batch
+        assert plan.chol_batch == 1 or plan.chol_batch * plan.chol_grid <= cus * 7 // 8, (r, batch)
+        plan.close()

@@ -64,13 +64,16 @@ def finishes(launches, rng, spread_set=True):
     workgroups end."""
     pend = [[[r for r in roles[x::NXCD] if r is not None and (spread_set or r[0] != "spread")] for x in range(NXCD)]
             for roles in launches]
+    place, done = {}, set()                # (launch, z) -> 'one' / 'spread'; factorisations that have ended
     need = [{} for _ in launches]          # workgroups of one set of matrix z
     for a, roles in enumerate(launches):
+        sets = {r[0] for r in roles if r is not None}
         for r in roles:
-            if r is not None and r[0] == "one":
+            if r is not None and r[0] == ("one" if "one" in sets else "spread"):
                 need[a][r[1]] = need[a].get(r[1], 0) + 1
+                if "one" not in sets:
+                    place[a, r[1]] = "spread"
     held = [[] for _ in range(NXCD)]       # (launch, role) resident
-    place, done = {}, set()                # (launch, z) -> 'one' / 'spread'; factorisations that have ended
 
     def settle():
         moved = True
@@ -145,3 +148,11 @@ def test_the_model_sees_the_starvation_without_the_spread_set():
     for slots in ((0, 0), (0, 1)):
         assert not all(finishes([launch(27, 1, NXCD, s, 48) for s in slots], random.Random(seed), spread_set=False)
                        for seed in range(40)), slots
+
+
+def test_two_of_the_widest_calls_must_be_ordered():
+    """the limit that spanqr.h states: 2048x1024 beside itself (99 workgroups and 128 of the solve, always spread) may
+    starve; beside a 768x512 call it does not"""
+    wide, call = launch(workgroups(32, 6), 1, 1, 0, 128), launch(27, 1, NXCD, 0, 48)
+    assert not all(finishes([wide, wide], random.Random(seed)) for seed in range(60))
+    assert all(finishes([wide, call], random.Random(seed)) for seed in range(12))
