@@ -3592,44 +3592,52 @@ int plan_device_setup(spanqr_plan* p, int device) {
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     p->cus = cus;
     // The owner part width and the placement. A factorisation wider than XCD_MIN_R whose workgroups all fit on one XCD
-    // goes there (m = NXCD); otherwise its workgroups are spread (m = 1). One matrix takes the narrowest parts, in tiles, that fit on
-    // one XCD with at most 8 tiles (12-tile parts there: 671 us per call at 3001 x 736, 6-tile parts spread: 656), or
-    // else OWNER_W; a batch the narrowest parts that run its Cholesky in the fewest launches. Each launch
+    // goes there (m = NXCD); otherwise its workgroups are spread (m = 1). One matrix takes the narrowest parts, in tiles,
+    // that fit on one XCD with at most 8 tiles (12-tile parts there: 671 us per call at 3001 x 736, 6-tile parts spread:
+    // 656), or else OWNER_W; a batch the narrowest parts that run its Cholesky in the fewest launches. Each launch
     // needs all its workgroups resident at once: several matrices take at most 7/8 of the device where each has an XCD
     // (28 CUs of each: a spread factorisation of another stream, four workgroups per XCD at r = 512, still fits beside
     // them) or three quarters of it spread (the margin leaves room for work of other streams).
+    // A batch of matrices that a single one would run spread (r > 608: on one XCD only with parts of more than 8 tiles) is
+    // spread where that takes parts of at most 8 tiles, unless only the one-XCD form leaves room for the solve in the same
+    // launch. Measured, one XCD / spread, us per call of n matrices of 2 r rows: r = 640 n = 2 545 / 542, n = 3 698 / 674,
+    // n = 4 868 / 853; 736 n = 3 996 / 952, n = 4 1105 / 1093; 800 n = 2 900 / 825; the solve beside it on one XCD only:
+    // 704 n = 2 613 / 672, 768 n = 2 728 / 768; more than 8 tiles in both forms: 640 n = 6 998 / 1043, 736 n = 7 1500 /
+    // 1572, 800 n = 4 1257 / 1295. Not so below: 768 x 512 n = 9 693 / 710 (16 tiles / 8), 1000 x 448 n = 10 723 / 758.
     {
-        const int widths[] = {OWNER_W, 8, 12, OWNER_WMAX};
-        int best_n = 1 << 30;
-        for (int pass = 0; pass < 2; ++pass)
-            for (int w : widths) {
-                int o = 0;
-                HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (const void*)k_chol<true, true>, 512, chol_lds_bytes(r, w)));
-                const int grid = chol_workgroups(r / CB, w), xcd = o * cus / NXCD;
-                int bmax;
-                if (pass == 0) {
-                    if (r <= XCD_MIN_R || grid > xcd || (p->batch == 1 && w > 8)) continue;
-                    // (the arrival words and both sets' call counters fit before the place word)
-                    if ((r / CB) * (r / CB + 1) + 3 * grid > PLACE_WORD) continue;
-                    bmax = std::max(1, std::min(NXCD * std::max(1, xcd * 7 / 8 / grid), o * cus * 7 / 8 / grid));
-                } else {
-                    if (p->batch == 1 && best_n == 1) break;
-                    if (o * cus < grid || (p->batch == 1 && w != OWNER_W)) continue;
-                    bmax = std::max(1, (o * cus * 3 / 4) / grid);
-                }
+        struct Form { int n, w, grid, m, bmax; };
+        Form best[2] = {{1 << 30, 0, 0, 0, 0}, {1 << 30, 0, 0, 0, 0}};   // on one XCD, spread
+        bool narrow_fits = false;   // on one XCD with parts of at most 8 tiles
+        for (int w : {OWNER_W, 8, 12, OWNER_WMAX}) {
+            int o = 0;
+            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, (const void*)k_chol<true, true>, 512, chol_lds_bytes(r, w)));
+            const int grid = chol_workgroups(r / CB, w), xcd = o * cus / NXCD;
+            narrow_fits |= w <= 8 && grid <= xcd;
+            auto offer = [&](Form& f, int m, int bmax) {
+                bmax = std::max(1, bmax);
                 const int launches = (p->batch + bmax - 1) / bmax;
-                if (launches < best_n) {
-                    best_n = launches;
-                    p->owner_w = w;
-                    p->chol_grid = grid;
-                    p->chol_m = pass == 0 ? NXCD : 1;
-                    p->chol_bmax = std::min(bmax, p->batch);
-                }
-            }
-        if (p->chol_m == NXCD) p->chol_slot = next_slot();
-        if (best_n == 1 << 30)
+                if (launches < f.n) f = {launches, w, grid, m, std::min(bmax, p->batch)};
+            };
+            // (the arrival words and both sets' call counters have to fit before the place word)
+            if (r > XCD_MIN_R && grid <= xcd && (p->batch > 1 || w <= 8) &&
+                (r / CB) * (r / CB + 1) + 3 * grid <= PLACE_WORD)
+                offer(best[0], NXCD, std::min(NXCD * std::max(1, xcd * 7 / 8 / grid), o * cus * 7 / 8 / grid));
+            if (o * cus >= grid && (p->batch > 1 || w == OWNER_W)) offer(best[1], 1, o * cus * 3 / 4 / grid);
+        }
+        const int rows = (p->K + 15) / 16;
+        auto solve_fits = [&](const Form& f) { return p->batch * (f.grid + rows) <= cus; };
+        bool spread = best[1].n < best[0].n;
+        if (best[1].n == best[0].n && !narrow_fits && best[1].w <= 8)
+            spread = !solve_fits(best[0]) || solve_fits(best[1]);
+        const Form& f = best[spread ? 1 : 0];
+        if (f.n == 1 << 30)
             return fail(SPANQR_EHIP, "the Cholesky needs %d co-resident workgroups, device holds too few",
                         chol_workgroups(r / CB, OWNER_WMAX));
+        p->owner_w = f.w;
+        p->chol_grid = f.grid;
+        p->chol_m = f.m;
+        p->chol_bmax = f.bmax;
+        if (f.m == NXCD) p->chol_slot = next_slot();
     }
     // The solve in the Cholesky's launch: enough rows per workgroup that one matrix's solve workgroups are resident
     // beside its Cholesky (one workgroup per CU: the launch's LDS is the Cholesky's); otherwise separate launches.

@@ -181,3 +181,17 @@ def test_batched_launches_leave_room(cuda, r):
         assert 1 <= plan.chol_batch <= batch
         assert plan.chol_batch == 1 or plan.chol_batch * plan.chol_grid <= cus * 7 // 8, (r, batch)
         plan.close()
+
+
+@pytest.mark.parametrize("K,r,n", [(700, 640, 3), (1472, 736, 2), (760, 736, 6)])
+def test_wide_batches(cuda, K, r, n):
+    """matrices that a single call spreads over the XCDs: a batch of them spread in narrow parts (640 x 3), one matrix per
+    XCD where only that leaves room for the solve in the launch (736 x 2), and where both forms take wide parts (736 x
+    6): the workgroups per matrix say which form ran, the bits are the single call's"""
+    Xs = [gen.bench_input(K, r, seed=s).to(cuda) for s in range(n)]
+    plan = get_plan(K, r, cuda, n)
+    assert (plan.chol_grid > 32) == (n == 3)
+    print(f"wide batch {n} x {K}x{r}", flush=True)
+    Qs = kcholqr_f_many(Xs)
+    for i in (0, n - 1):
+        assert_bits(Qs[i], kcholqr_f(Xs[i]), f"matrix {i} of {n} x {K}x{r} vs its single call")
