@@ -3213,8 +3213,9 @@ hipError_t trsm_limits(int maxsh) {
 
 // the fused instantiations: Q = 1 (r <= 256) with one row block, Q = 2 (r <= 512) with one or two, Q = 4
 // (r <= 1024) with one, and the wavefront-per-row-block solve (Q = 0) for r/32 = RB = 2, 4, 6, 8 column blocks
-// The hand-over protocols each is built for: the one for a single XCD (which also runs spread, as a batch may need it
-// at r = 192..512) and the one without it, for the widths where plans spread the factorisation.
+// The hand-over protocols each is built for: the one for a single XCD (which also runs spread, where a call settles for it
+// or, at r = 192..512, a batch is spread to need fewer launches: 17 matrices at r = 416) and the one without it, for
+// the widths where plans spread the factorisation.
 enum { FUSED_SPREAD = 1, FUSED_XCD = 2 };
 constexpr int fused_protocols(int q, int rb) {
     return q == 0 ? (rb >= 6 ? FUSED_XCD : FUSED_SPREAD) : q == 2 ? FUSED_XCD : FUSED_SPREAD | FUSED_XCD;
@@ -3386,7 +3387,7 @@ int launch_chol_solve(spanqr_plan* p, float alpha, float tau, float* scal, hipSt
         c.grid = p->chol_grid;
         c.m = p->chol_m;
         c.slot = p->chol_slot;
-        c.ticks = g_place_ticks;
+        c.ticks = p->chol_m == NXCD ? g_place_ticks : 0u;   // (spread from the start: nothing to wait for)
         c.ow = p->owner_w;
         c.lim = g_spin_limit;
         SolveArgs t{};

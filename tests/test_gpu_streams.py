@@ -1,13 +1,15 @@
 """Factorisations that prefer one XCD, where they cannot have it: with the wait for it set to nothing every call runs on
 the spread workgroups instead, bit-identical; and calls of two streams at once, which compete for the XCDs, end with the
 bits that each gives alone."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from spanqr_amd import _lib, borth, kchol, kcholqr_f, kcholqr_f_many, status
-from spanqr_amd.plan import get_plan
+from spanqr_amd.plan import Plan, get_plan, stream_handle
 from spanqr_amd.qrbench import gen
 
 from checks import assert_bits
@@ -48,6 +50,28 @@ def test_spread_set_of_a_batch(cuda, spread, K, r, n):
     torch.cuda.synchronize()
     for i in (0, n - 1):
         assert_bits(Qs[i], oracle.orth(Xs[i].numpy(), get_plan(K, r, cuda).split_rows), f"matrix {i} of the batch")
+
+
+def test_batch_plan_that_is_spread(cuda):
+    """17 matrices of 416 columns take one launch spread and two on XCDs of their own; called with two, the plan's solve
+    runs in the Cholesky's launch, whose kernel is the one-XCD one with no set on one XCD"""
+    K, r, n = 1000, 416, 2
+    Xs = [gen.bench_input(K, r, seed=i).to(cuda) for i in range(n)]
+    Qs = [torch.empty_like(X) for X in Xs]
+    plan = Plan(K, r, cuda.index, 17)
+    assert plan.chol_batch == 17
+
+    def arr(ts):
+        return (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
+
+    print(f"spread batch plan {n} of 17 x {K}x{r}", flush=True)
+    for _ in range(2):
+        _lib.check(_lib.lib().spanqr_orth_batched_f32(plan.handle, n, arr(Xs), r, arr(Qs), r, 5e-7, 1e-7, 1e-8, 2,
+                                                      stream_handle(cuda)))
+        torch.cuda.synchronize()
+        for X, Q in zip(Xs, Qs):
+            assert_bits(Q, oracle.orth(X.cpu().numpy(), plan.split_rows), "spread batch plan")
+    plan.close()
 
 
 @pytest.mark.parametrize("n", [192, 512, 608])
