@@ -250,10 +250,10 @@ int spanqr_plan_status(spanqr_plan* plan, void* stream);
 int spanqr_chol32(spanqr_plan* plan, const float* G, long ldg, const float* tau, float* L, long ldl, float* Li,
                   void* stream);
 
-/* Testing only (no counterpart in the reference): polls one bounded wait of the Cholesky makes before it gives up
+/* Testing only (no counterpart in the reference): polls one bounded wait of a Cholesky, fp32 or fp64, makes before it gives up
  * (default 2^20, about a second). Lowered to 0, a wait gives up unless its flag is already set, so the tests can
  * exercise the failure path with every kernel still ending normally: the wait-error word is set and the call's Q
- * comes out NaN. Applies to launches made after the call (a captured graph keeps the value it was captured with).
+ * comes out NaN (the fp64 factor is unspecified, and spanqr_chol64_status reports it). Applies to launches made after the call (a captured graph keeps the value it was captured with).
  * Not thread-safe with concurrent launches; restore the default (1048576) afterwards. */
 int spanqr_debug_spin_limit(unsigned polls);
 

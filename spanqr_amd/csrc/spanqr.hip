@@ -4938,7 +4938,7 @@ int spanqr_chol64(spanqr_chol64_plan* p, const double* G, long ldg, const double
         if (cap == hipStreamCaptureStatusNone) p->cleared.store(true);
     }
     k_chol64<<<chol_launch_size(p->grid, 1, p->m, 0), 512, chol64_lds_bytes(p->n, p->ow), st>>>(
-        G, ldg, p->n, tau, L, Li, Lf, Lif, p->flags, p->grid, p->m, p->slot, p->ow, SPIN_LIMIT, g_place_ticks);
+        G, ldg, p->n, tau, L, Li, Lf, Lif, p->flags, p->grid, p->m, p->slot, p->ow, g_spin_limit, g_place_ticks);
     HIPCHK(hipGetLastError());
     return SPANQR_OK;
 }

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from spanqr_amd import _lib, borth, kcholqr_f, kcholqr_f_many, set_checked, stages, status
+from spanqr_amd import _lib, borth, kchol, kcholqr_f, kcholqr_f_many, set_checked, stages, status
 from spanqr_amd.plan import get_plan
 from spanqr_amd.qrbench import gen
 
@@ -110,3 +110,28 @@ def test_blocked_give_up_is_reported(cuda):
     Q1 = borth(Xd, 256)
     status(Xd)
     assert_bits(Q1, Q0, "blocked call after the failure vs before")
+
+
+@pytest.mark.parametrize("n", [512, 640])   # on one XCD, spread over the device
+def test_chol64_give_up_is_reported(cuda, n):
+    """the fp64 Cholesky's status reports a wait that gave up, in the call it happened in only; the flags only count up, so
+    the next call on the same plan is whole again without a clear"""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n + 20, n))
+    G = torch.from_numpy(X.T @ X).to(cuda)
+    want = oracle.chol64(X.T @ X, 1e-12)
+    kchol.chol64(G, 1e-12)
+    kchol.status(n, cuda)
+    for _ in range(2):
+        print(f"failure path: chol64 n={n}, spin limit 0", flush=True)
+        _lib.lib().spanqr_debug_spin_limit(0)
+        try:
+            kchol.chol64(G, 1e-12)
+            with pytest.raises(_lib.SpanqrError, match="exceeded its bound"):
+                kchol.status(n, cuda)
+        finally:
+            _lib.lib().spanqr_debug_spin_limit(DEFAULT_LIMIT)
+        out = kchol.chol64(G, 1e-12)
+        kchol.status(n, cuda)
+        for x, y, what in zip(out, want, ("L", "Li", "Lf", "Lif")):
+            assert np.array_equal(x.cpu().numpy(), y), f"chol64 {what} after the failure"
