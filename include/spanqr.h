@@ -58,7 +58,8 @@ enum {
     SPANQR_Q_R = 1,
     SPANQR_Q_SPLITS = 2,         /* Gram row splits S */
     SPANQR_Q_SPLIT_ROWS = 3,     /* rows per split KS (a multiple of 32) */
-    SPANQR_Q_CHOL_GRID = 4,      /* workgroups of one matrix's Cholesky (max(1, r/32 - 3)) */
+    SPANQR_Q_CHOL_GRID = 4,      /* workgroups of one matrix's Cholesky: one for the diagonal, the parts of
+                                    tile rows 4 to r/32 - 1 */
     SPANQR_Q_WORKSPACE_MB = 5,   /* workspace size, MiB (rounded up) */
     SPANQR_Q_DEVICE = 6,
     SPANQR_Q_BATCH = 7,          /* matrices per call the plan holds workspace for */

@@ -1441,7 +1441,7 @@ size_t chol_lds_bytes(int r, int w) {
 // npart[l], npart[l + 64], ... in order, then a shift-down tree over the 64 lane sums; nrm = sqrtf(fp32(sum)),
 // shift = alpha * nrm added to the diagonal after the first load, tau = tau_rel * nrm + 1e-30 (kcholqr.py:107-109).
 // flags: [nb * nb] panel flags (L(i, j) published; (j, j): L(j, j) and Li_j), [nb] hand-over flags (tile row i),
-// [64] per-workgroup call counters. STAMP: workgroup 0 records the wall clock at 1 + 4j + s for step j: s = 0 step
+// per-workgroup call counters, arrival words and the call's place (FLAG_STRIDE). STAMP: workgroup 0 records the wall clock at 1 + 4j + s for step j: s = 0 step
 // start, 1 step end, 2 look-ahead done, 3 tile factor done; slot 0 is the kernel start, 1 + 4 nb the end;
 // 2 + 4 nb + j: wave 1's row work of step j done; 2 + 5 nb + j: wave 3's done; 2 + 6 nb + j: the hand-over of row j+2
 // seen; 2 + 7 nb + j: row j+2 fetched; 2 + 8 nb + j: its panel L(j+2, j-1) formed; 2 + 9 nb + j: wave 2 done;
@@ -3787,7 +3787,11 @@ void project(const spanqr_plan* p, const float* Q, long ldq, int j, const float*
         // A workgroup per tile, or per quadrant where whole tiles would load the CUs unevenly (by more than a quarter):
         // at K = 17408, 256 columns, us per launch, tiles / quadrants: j = 256 25 / 30, 512 45 / 54, 1024 86 / 103 (512
         // tiles and splits on 256 CUs: even), 768 82 / 79 (528), 1280 135 / 122 (560), 1536 152 / 142 (576), 1792 184 /
-        // 168 (560). k_gram, for all of them: 26, 49, 94, 91, 146, 170, 202.
+        // 168 (560). k_gram, for all of them: 26, 49, 94, 91, 146, 170, 202. Other widths and heights, one product per
+        // call of borth without reorth, us per call: even loads (512) 17408 x 1024 in blocks of 512 2613 / 2643, 17408 x
+        // 2048 of 1024 8600 / 8715, 6000 x 1024 of 512 1125 / 1133; uneven 17408 x 1536 of 768 (576) 5444 / 5408, 9000 x
+        // 1280 of 640 (600) 2550 / 2539, 9000 x 1152 of 384 (540, 576) 1968 / 1960, 12000 x 576 of 192 (522) 1014 / 1008,
+        // level at 17408 x 960 of 320 (525, 550) and 6000 x 768 of 384 (540).
         const long cus = p->blk->cus, wgs = (long)U * S;
         const bool quads = (wgs + cus - 1) / cus * cus * 4 > wgs * 5;
         k_gramr<true><<<dim3(quads ? 4 * U : U, S), quads ? 64 : 256, 0, st>>>(P, ldq, p->K, 0, KS, p->Tp, j, Cin, ldc,

@@ -75,11 +75,11 @@ def test_chol64_rejects_bad_inputs(cuda):
         kchol.chol64(torch.zeros(1056, 1056, device=cuda, dtype=torch.float64), 1e-9)
 
 
-@pytest.mark.parametrize("n", [96, 192, 224, 544, 608, 640, 992])
+@pytest.mark.parametrize("n", [96, 192, 224, 544, 576, 608, 640, 992])
 def test_chol64_row_parts(cuda, n):
     """the sizes where the split changes: the first tile row with a workgroup of its own (96), rows of one and of two
-    parts (192, 224), the wider parts that still fit on one XCD (544, 608), the workgroups spread over the device
-    (640, 992), with an ill-scaled G and with a pivot row that vanishes in the last tile"""
+    parts (192, 224), a whole XCD in the narrow parts (544), the wider parts that still fit on one (576, 608), the
+    workgroups spread over the device (640, 992), with an ill-scaled G and with a pivot row that vanishes in the last tile"""
     rng = np.random.default_rng(n)
     X = rng.standard_normal((n + 9, n)) * np.exp(rng.uniform(-6, 6, n))
     X[:, n - 2] = X[:, 1]
