@@ -10,7 +10,6 @@ import pytest
 from spanqr_amd import _lib
 
 NXCD, CUS = 8, 32   # XCDs, compute units of each (a workgroup's LDS leaves room for one per unit)
-NOTHING = 1 << 20
 
 
 def workgroups(nb, w, first=4):
