@@ -3598,7 +3598,9 @@ int plan_device_setup(spanqr_plan* p, int device) {
     // 656), or else OWNER_W; a batch the narrowest parts that run its Cholesky in the fewest launches. Each launch
     // needs all its workgroups resident at once: several matrices take at most 7/8 of the device where each has an XCD
     // (28 CUs of each: a spread factorisation of another stream, four workgroups per XCD at r = 512, still fits beside
-    // them) or three quarters of it spread (the margin leaves room for work of other streams).
+    // them) or three quarters of it spread (the margin leaves room for work of other streams). What the room costs where
+    // eight matrices would take 29 to 31 CUs of each XCD, eight of 2 r rows per call, in one launch without it / now: r =
+    // 544 912 / 925 us (8-tile parts), 736 1597 / 1605 (16-tile), 768 1700 / 2090 and 800 1979 / 2422 (two launches).
     // A batch of matrices that a single one would run spread (r > 608: on one XCD only with parts of more than 8 tiles) is
     // spread where that takes parts of at most 8 tiles, unless only the one-XCD form leaves room for the solve in the same
     // launch. Measured, one XCD / spread, us per call of n matrices of 2 r rows: r = 640 n = 2 545 / 542, n = 3 698 / 674,
